@@ -135,221 +135,386 @@ __global__ __launch_bounds__(256) void fw_rmsnorm_kernel(const float * x, const 
     }
 }
 
-/* Rope, the KV store and attention over the layer's window of the cache,
- * positions start .. pos (model.rs:484-557; window 0: every position), split
- * by positions so that a long window keeps many CUs busy:
+/* ---- attention of one token, or of a verify block of up to 8 ----
+ * Softmax attention over the layer's window of the cache (model.rs:505-557;
+ * window 0: every position), split by positions over workgroups whose
+ * partial results a second launch combines:
  *
- *   fw_attn_part_kernel: workgroup (chunk, kv head), one wave per query head
- *     of the kv head's group, kAttnChunk positions. Each lane holds VPL
- *     consecutive elements of a head. The wave rotates its query head in
- *     registers (rope over the first pdim elements with the position's f32
- *     table, model.rs:416-428, which the state kernel computes once per token
- *     for each layer type; the pair partner of element e is e +- pdim/2, in the
- *     lane pdim/2/VPL away, fetched with a lane permute). The chunk holding
- *     pos rotates the new key the same way, uses it and the new value from
- *     registers, and its first wave stores both in the cache (model.rs:
- *     498-503); other chunks read only older rows. A score is a lane-local dot
- *     and a butterfly; the wave keeps its chunk's maximum m, sum
- *     l = sum_j e^(s_j - m) and unnormalized o = sum_j e^(s_j - m) V[j].
- *   fw_attn_combine_kernel: workgroup per query head; rescales the chunks to
- *     the overall maximum M, divides by L = sum_c l_c e^(m_c - M) and applies
- *     the head's sigmoid gate. Its four waves take every fourth chunk.
+ *   fw_attn_split_kernel: workgroup (split, kv head). The window's positions
+ *     are cut into tiles of 16 and split s takes `per` consecutive tiles,
+ *     per = ceil(tiles / nsplit): one tile each up to 16 * nsplit positions,
+ *     so a short window still spreads over the chip, and a long one costs
+ *     nsplit partials per head whatever its length. All the columns that read
+ *     a kv head's rows run together: column t * G + g is token t (of N) and
+ *     query head g of the group's G, at most 32, in NB blocks of 16. So K and
+ *     V cross HBM once per call, on the f32 matrix cores.
+ *   fw_attn_combine_kernel: per (head, token), rescales the partials to their
+ *     overall reference M, divides by L = sum_s l_s e^(m_s - M) and applies the
+ *     head's sigmoid gate.
  *
- * That is the CPU's softmax with the sum regrouped by chunk. Launch shapes
- * are fixed (the longest window), so a captured graph serves every position:
- * chunks past the current window do nothing. */
-constexpr int kAttnChunk = 16;
+ * The split kernel's four waves share each tile by head elements: wave w
+ * contracts elements DW w .. DW w + DW - 1 (DW = HD / 4) of K against Q
+ * (S^T = K Q^T, positions x columns), the four partial scores meet in LDS
+ * (one barrier per tile, two buffers), every wave forms the same weights and
+ * adds its own elements of O^T += V^T P^T. So one tile takes a quarter of a
+ * wave's matrix time, which a short window needs, and a wave holds only
+ * DW / 2 registers per tile of K and V, which lets the next tile be in flight
+ * under this one, which a long window needs (two tiles ahead: 45.3 -> 47.0 us
+ * at 30000 positions, 22.7 -> 24.9 for the block below).
+ *
+ * Operand layout (lane 16 g + c), as in the prompt kernel below: a lane
+ * reads its K row c as runs of 4 elements (k-step ks contracts element
+ * 16 (ks / 4) + 4 g + ks % 4 of the wave's range), holds the scores of
+ * positions 4 g + i for column c, and reads elements VW c .. + VW - 1
+ * (VW = DW / 16) of the V rows 4 g + ks: O^T block r holds element
+ * VW (4 g + i) + r of column c.
+ *
+ * The weights are exp(score - m) for a reference m per column that moves only
+ * when a score passes it by more than kPaLag (the prompt kernel's rule): the
+ * quotient does not depend on m, and most tiles skip the rescale.
+ *
+ * DEC (one decode token): position and rope tables come from device memory
+ * (the state kernel's), the kernel rotates its query heads itself, and the
+ * split whose tile ends at pos rotates the new key, uses it and the new value
+ * from LDS, and stores both in the cache (model.rs:498-503); no other split
+ * reads row pos, which before the store may hold anything. The launch shape
+ * is fixed by the longest window, so a captured graph serves every position:
+ * splits past the current window do nothing.
+ *
+ * Otherwise (a block): queries and keys are rotated and every key and value
+ * is in the cache. A tile that some column sees only in part (causal end or
+ * window start) must not weight a hidden V row by zero when it holds an
+ * infinity or NaN; such a tile adds its rows one by one instead.
+ *
+ * What bounds it: HBM at long context (8 KB per position, read once, 5.2
+ * TB/s); latency at short. Measured with four kv heads of 256 elements
+ * (before: a workgroup per 16 positions, a wave per query head and token, all
+ * partials combined by four waves per head): one token at position 30007 70 +
+ * 56 -> 47 + 4.7 us (partials + combine), at 1003 9.4 + 4.7 -> 7.4 + 4.6, a
+ * 512-position window 7.5 + 4.7 -> 6.1 + 4.6; a block of 8 at 6001 79 + 13 ->
+ * 22 + 4.0, its 512-position windows 10.2 + 4.8 -> 9.0 + 4.0.
+ * kAttnSplits: 64 against 128 costs the split kernel 1.7 us at 30007 and saves
+ * every combine 0.6; 256 splits 54 + 6.3 at 30007. */
+constexpr int kAttnChunk = 16;     /* positions per tile */
+constexpr int kAttnSplits = 64;    /* partials per head and token, at most */
+constexpr float kPaLag = 8.0f;     /* how far a score may pass the reference maximum */
 
-template <int VPL>
-__global__ __launch_bounds__(256) void fw_attn_part_kernel(const float * qkv, int qd, int kvd, float * kc, float * vc,
-                                                            const int * st, int window, int heads, int kv_heads,
-                                                            int pdim, const float * rtab, float scale, int nch_max,
-                                                            float * part) {
-    constexpr int hd = 64 * VPL, C = kAttnChunk;
-    typedef float fv __attribute__((ext_vector_type(VPL)));
-    const int pos = st[1];
-    const int start = window > 0 && pos + 1 > window ? pos + 1 - window : 0;
-    const int n = pos + 1 - start;
-    const int chunk = blockIdx.x, kvh = blockIdx.y;
-    const int G = heads / kv_heads;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int j0 = chunk * C;
-    if (j0 >= n) return;                        /* uniform: the combine reads chunks < ceil(n / chunk) */
-    const int jn = min(C, n - j0);
-    const int h = kvh * G + wave;               /* h * kv_heads / heads == kvh */
-    const int half = pdim / 2;                  /* a multiple of VPL (the host checks) */
-    /* x rotated by position pos: element e < half pairs with e + half,
-     * e in [half, pdim) with e - half (apply_rope, model.rs:430-438). The
-     * lane's cos and sin are read unconditionally (elements past pdim read
-     * entry 0 and do not use it) and before the K and V rows: read inside
-     * the per-element branch, each took a memory round trip of its own,
-     * after the query's, ahead of the rows' loads. */
-    const int e0 = lane * VPL;
-    fv cv, sv;
+struct AttnArgs {
+    const float * qkv;   /* [N][ldq]: q, k, v of each token */
+    float * kc, * vc;    /* the layer's cache rows [max_ctx][kvd] */
+    const int * st;      /* DEC: token, position */
+    const float * rtab;  /* DEC: the position's rope table [cos, sin][128] */
+    float * po, * pml;   /* partials: [N * heads][nsplit][HD], [N * heads][nsplit][m, l] */
+    int ldq, qd, kvd, pos0, N, window, heads, kv_heads, pdim, nsplit;
+    float scale;
+};
+
+/* the splits of a window of n positions: tiles per split */
+__host__ __device__ __forceinline__ int attn_per(int n, int nsplit) {
+    const int tiles = (n + kAttnChunk - 1) / kAttnChunk;
+    return (tiles + nsplit - 1) / nsplit;
+}
+
+template <int HD, int NB, int DEC>
+__global__ __launch_bounds__(256, 2) void fw_attn_split_kernel(const AttnArgs A) {
+    constexpr int DW = HD / 4, KQ = DW / 16, VW = DW / 16, QS = HD + 4;
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    typedef float vv __attribute__((ext_vector_type(VW)));
+    __shared__ __attribute__((aligned(16))) float lq[NB * 16 * QS];
+    __shared__ f4v ls[2][4][NB][64];
+    __shared__ __attribute__((aligned(16))) float lkv[DEC ? 2 * HD : 4];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, c = lane & 15;
+    const int pos = DEC ? A.st[1] : A.pos0, N = DEC ? 1 : A.N, kvh = blockIdx.y;
+    const int G = A.heads / A.kv_heads, kvd = A.kvd;
+    const int pfirst = A.window > 0 && pos + 1 > A.window ? pos + 1 - A.window : 0;
+    const int plast = pos + N - 1, n = plast - pfirst + 1;
+    const int per = attn_per(n, A.nsplit), ntile = (n + kAttnChunk - 1) / kAttnChunk;
+    const int tb = blockIdx.x * per, te = min(tb + per, ntile);
+    if (tb >= ntile) return;   /* uniform: the combine reads splits < ceil(ntile / per) */
+    const bool newest = DEC && te == ntile;
+    /* rows past the last stored one repeat it */
+    const int rlast = DEC ? max(pos - 1, 0) : plast;
+    const int d0 = DW * wave;
+    const float * kb = A.kc + (size_t) kvh * HD + d0 + 4 * g;
+    const float * vb = A.vc + (size_t) kvh * HD + d0 + VW * c;
+    f4v kf[2][KQ];
+    vv vf[2][4];
+    auto fetch = [&](int tile, int s) {
+        const int p = pfirst + kAttnChunk * min(tile, te - 1);
+        const float * kp = kb + (size_t) min(p + c, rlast) * kvd;
 #pragma unroll
-    for (int v = 0; v < VPL; v++) {
-        const int e = e0 + v;
-        const int i = e < half ? e : (e < 2 * half ? e - half : 0);
-        cv[v] = rtab[i];
-        sv[v] = rtab[128 + i];
-    }
-    auto rope = [&](fv x) -> fv {
-        const int pl = e0 < half ? lane + half / VPL : (e0 < pdim ? lane - half / VPL : lane);
-        fv p, r = x;
+        for (int j = 0; j < KQ; j++) kf[s][j] = *(const f4v *) (kp + 16 * j);
 #pragma unroll
-        for (int v = 0; v < VPL; v++) p[v] = __shfl(x[v], pl, 64);
-#pragma unroll
-        for (int v = 0; v < VPL; v++) {
-            const int e = e0 + v;
-            if (e < 2 * half) r[v] = e < half ? x[v] * cv[v] - p[v] * sv[v] : x[v] * cv[v] + p[v] * sv[v];
-        }
-        return r;
+        for (int ks = 0; ks < 4; ks++) vf[s][ks] = *(const vv *) (vb + (size_t) min(p + 4 * g + ks, rlast) * kvd);
     };
-    const fv qx = *(const fv *) (qkv + (size_t) h * hd + lane * VPL);
-    const float * kb = kc + (size_t) (start + j0) * kvd + (size_t) kvh * hd + lane * VPL;
-    const float * vb = vc + (size_t) (start + j0) * kvd + (size_t) kvh * hd + lane * VPL;
-    /* every K and V row of the chunk requested at once (rows past the
-     * window re-read the last one and get weight zero), then the query
-     * rotated while they are in flight */
-    fv kr[C], vr[C];
+    fetch(tb, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    /* the queries (rows past the last column repeat it) */
+    const int ncol = N * G;
+    if constexpr (DEC) {
+        /* rotated here (model.rs:416-438): element e < half pairs with
+         * e + half, e in [half, 2 half) with e - half */
+        const int half = A.pdim / 2, rows = newest ? G + 2 : G;
+        constexpr int PER = (6 * HD + 255) / 256;   /* G <= 4 query rows, the new key and value */
+        float x[PER], y[PER], cs[PER], sn[PER];
 #pragma unroll
-    for (int j = 0; j < C; j++) kr[j] = *(const fv *) (kb + (size_t) min(j, jn - 1) * kvd);
+        for (int k = 0; k < PER; k++) {
+            const int i = tid + 256 * k, r = min(i / HD, rows - 1), e = i & (HD - 1);
+            const float * src = A.qkv + (r < G ? (size_t) (kvh * G + r) * HD : (size_t) A.qd + (size_t) (r - G) * kvd + (size_t) kvh * HD);
+            const int q = e < half ? e : (e < 2 * half ? e - half : 0);
+            x[k] = src[e];
+            y[k] = src[e < half ? e + half : (e < 2 * half ? e - half : e)];
+            cs[k] = A.rtab[q];
+            sn[k] = A.rtab[128 + q];
+        }
 #pragma unroll
-    for (int j = 0; j < C; j++) vr[j] = *(const fv *) (vb + (size_t) min(j, jn - 1) * kvd);
-    const fv q = rope(qx);
-    if (j0 + jn == n) {
-        /* this chunk ends at pos: the new key and value, from qkv */
-        const fv kn = rope(*(const fv *) (qkv + qd + (size_t) kvh * hd + lane * VPL));
-        const fv vn = *(const fv *) (qkv + qd + kvd + (size_t) kvh * hd + lane * VPL);
+        for (int k = 0; k < PER; k++) {
+            const int i = tid + 256 * k, r = i / HD, e = i & (HD - 1);
+            if (r >= rows) continue;
+            float v = x[k];
+            if (r <= G && e < 2 * half) v = e < half ? x[k] * cs[k] - y[k] * sn[k] : x[k] * cs[k] + y[k] * sn[k];
+            if (r < G) {
+                lq[r * QS + e] = v;
+            } else {
+                lkv[(r - G) * HD + e] = v;
+                float * dst = r == G ? A.kc : A.vc;
+                dst[(size_t) pos * kvd + (size_t) kvh * HD + e] = v;
+            }
+        }
+    } else {
 #pragma unroll
-        for (int j = 0; j < C; j++)
-            if (j == jn - 1) { kr[j] = kn; vr[j] = vn; }
-        if (wave == 0) {
-            *(fv *) (kc + (size_t) pos * kvd + (size_t) kvh * hd + lane * VPL) = kn;
-            *(fv *) (vc + (size_t) pos * kvd + (size_t) kvh * hd + lane * VPL) = vn;
+        for (int k = 0; k < NB * 16 * HD / 4 / 256; k++) {
+            const int i = tid + 256 * k, col = min(i / (HD / 4), ncol - 1), e = 4 * (i & (HD / 4 - 1));
+            const int t = col / G, h = kvh * G + col - t * G;
+            *(f4v *) (lq + (i / (HD / 4)) * QS + e) = *(const f4v *) (A.qkv + (size_t) t * A.ldq + (size_t) h * HD + e);
         }
     }
-    float sc[C];
-    float m = -INFINITY;
+    __syncthreads();
+    float qv[NB][4 * KQ];
+    int pos_t[NB], start_t[NB];
 #pragma unroll
-    for (int j = 0; j < C; j++) {
-        float s = 0.0f;
+    for (int b = 0; b < NB; b++) {
+        const int col = min(16 * b + c, ncol - 1);
 #pragma unroll
-        for (int v = 0; v < VPL; v++) s += q[v] * kr[j][v];
+        for (int j = 0; j < KQ; j++) {
+            const f4v q4 = *(const f4v *) (lq + (DEC ? col : 16 * b + c) * QS + d0 + 16 * j + 4 * g);
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-        sc[j] = s * scale;
-        if (j < jn) m = fmaxf(m, sc[j]);
+            for (int i = 0; i < 4; i++) qv[b][4 * j + i] = q4[i];
+        }
+        pos_t[b] = pos + col / G;
+        start_t[b] = A.window > 0 && pos_t[b] + 1 > A.window ? pos_t[b] + 1 - A.window : 0;
     }
-    float l = 0.0f;
-    fv o = (fv) 0.0f;
+    /* positions every column sees: the tiles inside need no mask */
+    const int allfirst = A.window > 0 && plast + 1 > A.window ? plast + 1 - A.window : 0;
+    f4v o[NB][VW];
+    float m[NB], l[NB];
 #pragma unroll
-    for (int j = 0; j < C; j++) {
-        /* rows past jn are padding that may hold anything (the row at pos
-         * before its store): skipped, not weighted by zero */
-        if (j < jn) {
-            const float e = expf(sc[j] - m);
-            l += e;
-            o += e * vr[j];
+    for (int b = 0; b < NB; b++) {
+        m[b] = -INFINITY;
+        l[b] = 0.0f;
+#pragma unroll
+        for (int r = 0; r < VW; r++) o[b][r] = f4v{0.f, 0.f, 0.f, 0.f};
+    }
+    auto step = [&](int tile, int s) {
+        const int p = pfirst + kAttnChunk * tile;
+        const bool edge = p + kAttnChunk > pos + (DEC ? 0 : 1) || p < allfirst;   /* uniform */
+        if (DEC && edge) {
+            /* the last tile: rows from pos on are the new key and value */
+            if (p + c >= pos) {
+#pragma unroll
+                for (int j = 0; j < KQ; j++) kf[s][j] = *(const f4v *) (lkv + d0 + 16 * j + 4 * g);
+            }
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++)
+                if (p + 4 * g + ks >= pos) vf[s][ks] = *(const vv *) (lkv + HD + d0 + VW * c);
+        }
+        /* this wave's elements of S^T, two chains per block */
+        f4v sa[NB], sb[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) sa[b] = sb[b] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < KQ; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2)
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    sa[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s][j][i], qv[b][4 * j + i], sa[b], 0, 0, 0);
+                    sb[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s][j][i + 1], qv[b][4 * j + i + 1], sb[b], 0, 0, 0);
+                }
+#pragma unroll
+        for (int b = 0; b < NB; b++) ls[s][wave][b][lane] = sa[b] + sb[b];
+        __syncthreads();
+        float e[NB][4];
+        bool over = false;
+        float mc[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const f4v sc = (ls[s][0][b][lane] + ls[s][1][b][lane]) + (ls[s][2][b][lane] + ls[s][3][b][lane]);
+            mc[b] = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int pp = p + 4 * g + i;
+                e[b][i] = !edge || (pp >= start_t[b] && pp <= pos_t[b]) ? sc[i] * A.scale : -INFINITY;
+                mc[b] = fmaxf(mc[b], e[b][i]);
+            }
+            over = over || mc[b] > m[b] + kPaLag;
+        }
+        if (__any(over)) {   /* uniform, and the same in every wave */
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                float x = fmaxf(mc[b], __shfl_xor(mc[b], 16, 64));
+                x = fmaxf(x, __shfl_xor(x, 32, 64));
+                const float mn = fmaxf(m[b], x);
+                const float a = mn == -INFINITY ? 1.0f : expf(m[b] - mn);   /* nothing seen yet: no rescale */
+                l[b] *= a;
+#pragma unroll
+                for (int r = 0; r < VW; r++) o[b][r] *= a;
+                m[b] = mn;
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                e[b][i] = e[b][i] == -INFINITY ? 0.0f : expf(e[b][i] - m[b]);
+                l[b] += e[b][i];
+            }
+        if constexpr (!DEC) {
+            bool bad = false;
+            if (edge) {
+#pragma unroll
+                for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+                    for (int r = 0; r < VW; r++) bad = bad || !__builtin_isfinite(vf[s][ks][r]);
+            }
+            if (edge && __any(bad)) {
+                /* a hidden row may hold an infinity or NaN: row by row, hidden rows left out */
+#pragma unroll 1
+                for (int q = 0; q < 4; q++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const int pp = p + 4 * q + k;
+                        const float * vr = A.vc + (size_t) min(pp, rlast) * kvd + (size_t) kvh * HD + d0 + 4 * VW * g;
+#pragma unroll
+                        for (int b = 0; b < NB; b++) {
+                            const float w = __shfl(e[b][k], 16 * q + c, 64);
+                            if (pp >= start_t[b] && pp <= pos_t[b])
+#pragma unroll
+                                for (int i = 0; i < 4; i++)
+#pragma unroll
+                                    for (int r = 0; r < VW; r++) o[b][r][i] += w * vr[VW * i + r];
+                        }
+                    }
+                return;
+            }
+        }
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+            for (int r = 0; r < VW; r++)
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+                    o[b][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[s][ks][r], e[b][ks], o[b][r], 0, 0, 0);
+    };
+    /* tile t in slot and score buffer (t - tb) & 1, the next one requested
+     * before it is worked (past the end the last one again: a branch between
+     * the loads would make the waits for this tile cover them too) */
+    for (int t = tb; t < te;) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            if (t < te) {
+                __builtin_amdgcn_sched_barrier(0);
+                fetch(t + 1, u ^ 1);
+                __builtin_amdgcn_sched_barrier(0);
+                step(t, u);
+            }
+            t++;
         }
     }
-    float * P = part + ((size_t) h * nch_max + chunk) * (hd + 2);
-    *(fv *) (P + lane * VPL) = o;
-    if (lane == 0) {
-        P[hd] = m;
-        P[hd + 1] = l;
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        l[b] += __shfl_xor(l[b], 16, 64);
+        l[b] += __shfl_xor(l[b], 32, 64);
+        const int col = 16 * b + c;
+        if (col >= ncol) continue;
+        const int t = col / G, h = kvh * G + col - t * G;
+        const size_t at = ((size_t) t * A.heads + h) * A.nsplit + blockIdx.x;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            vv v;
+#pragma unroll
+            for (int r = 0; r < VW; r++) v[r] = o[b][r][i];
+            *(vv *) (A.po + at * HD + d0 + VW * (4 * g + i)) = v;
+        }
+        if (wave == 0 && g == 0) {
+            A.pml[2 * at] = m[b];
+            A.pml[2 * at + 1] = l[b];
+        }
     }
 }
 
-/* The combine of one query head from its nch chunk partials P (o, m, l per
- * chunk at stride hd + 2), four waves: M = max m_c, L = sum_c l_c e^(m_c - M)
- * (threads over chunks), wave w summing e^(m_c - M) o_c over chunks w,
- * w + 4, ... in increasing order, then out = the waves' sum / L times the
- * head's sigmoid gate gl. Each wave's first kPre chunk vectors are requested
- * before the m_c reductions, so up to 4 * kPre chunks cost one memory round
- * trip (a wave had taken one or four chunks per round trip: at context 1024
- * five of them). wts: 2 * nch floats of dynamic LDS. */
+/* The combine of (head blockIdx.x, token blockIdx.y): M = max m_s, L = sum_s
+ * l_s e^(m_s - M), wave w summing e^(m_s - M) o_s over splits
+ * w, w + 8, ... in increasing order, then the waves' sums in wave order, over
+ * L, times the head's sigmoid gate. All of the partials' vectors that a wave
+ * needs are requested at once (kPre each, kAttnSplits in all), behind the m
+ * and l loads whose reductions they overlap: one memory round trip. */
 template <int VPL>
-__device__ __forceinline__ void attn_combine_head(const float * P, int nch, float gl, float * out, uint16_t * out16,
-                                                  float * wts) {
-    constexpr int hd = 64 * VPL, kPre = 20;
+__global__ __launch_bounds__(512) void fw_attn_combine_kernel(const AttnArgs A, int dec, const float * gate, int ldg,
+                                                              float * out, uint16_t * out16) {
+    constexpr int HD = 64 * VPL, W = 8, kPre = kAttnSplits / W;
     typedef float fv __attribute__((ext_vector_type(VPL)));
-    __shared__ float red[8];
-    __shared__ fv acc[4][64];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    float * ls = wts + nch;
-    float M = -INFINITY;
-    for (int c = t; c < nch; c += 256) {
-        const float mc = P[(size_t) c * (hd + 2) + hd], lc = P[(size_t) c * (hd + 2) + hd + 1];
-        wts[c] = mc;
-        ls[c] = lc;
-        M = fmaxf(M, mc);
+    __shared__ float wts[kAttnSplits];
+    __shared__ fv acc[W][64];
+    __shared__ float red;
+    const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const float gl = gate[(size_t) t * ldg + h];
+    const int pos = dec ? A.st[1] : A.pos0, N = dec ? 1 : A.N;
+    const int pfirst = A.window > 0 && pos + 1 > A.window ? pos + 1 - A.window : 0;
+    const int n = pos + N - pfirst, per = attn_per(n, A.nsplit);
+    const int ns = ((n + kAttnChunk - 1) / kAttnChunk + per - 1) / per;
+    const size_t row = (size_t) t * A.heads + h, at = row * A.nsplit;
+    static_assert(kAttnSplits == 64, "wave 0 holds one split per lane");
+    float mc = -INFINITY, lc = 0.0f;
+    if (tid < ns) {
+        mc = A.pml[2 * (at + tid)];
+        lc = A.pml[2 * (at + tid) + 1];
     }
-    const float * Pl = P + lane * VPL;
     fv pre[kPre];
+    const float * P = A.po + at * HD + lane * VPL;
 #pragma unroll
-    for (int k = 0; k < kPre; k++) {
-        /* chunks past nch re-read the last one (no branch between the
-         * loads) and are not added. After the m_c loads on purpose: their
-         * round trip then overlaps the reductions below (issued first, all
-         * of them waited for together: decode token 2093 -> 2111 us) */
-        const int c = min(wave + 4 * k, nch - 1);
-        pre[k] = *(const fv *) (Pl + (size_t) c * (hd + 2));
+    for (int k = 0; k < kPre; k++) pre[k] = *(const fv *) (P + (size_t) min(wave + W * k, ns - 1) * HD);
+    if (wave == 0) {
+        float M = mc;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+        const float w = tid < ns ? expf(mc - M) : 0.0f;
+        wts[tid] = w;
+        float L = w * lc;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o, 64);
+        if (lane == 0) red = L;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
-    if (lane == 0) red[wave] = M;
-    __syncthreads();
-    M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    float L = 0.0f;
-    for (int c = t; c < nch; c += 256) {
-        const float w = expf(wts[c] - M);
-        wts[c] = w;
-        L += w * ls[c];
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o, 64);
-    if (lane == 0) red[4 + wave] = L;
     __syncthreads();
     fv o = (fv) 0.0f;
 #pragma unroll
     for (int k = 0; k < kPre; k++)
-        if (wave + 4 * k < nch) o += wts[wave + 4 * k] * pre[k];
-    int c = wave + 4 * kPre;
-    for (; c + 12 < nch; c += 16) {
-        const fv a0 = *(const fv *) (Pl + (size_t) c * (hd + 2)), a1 = *(const fv *) (Pl + (size_t) (c + 4) * (hd + 2));
-        const fv a2 = *(const fv *) (Pl + (size_t) (c + 8) * (hd + 2)), a3 = *(const fv *) (Pl + (size_t) (c + 12) * (hd + 2));
-        o += wts[c] * a0;
-        o += wts[c + 4] * a1;
-        o += wts[c + 8] * a2;
-        o += wts[c + 12] * a3;
-    }
-    for (; c < nch; c += 4) o += wts[c] * *(const fv *) (Pl + (size_t) c * (hd + 2));
+        if (wave + W * k < ns) o += wts[wave + W * k] * pre[k];
     acc[wave][lane] = o;
     __syncthreads();
     if (wave == 0) {
-        const float inv = 1.0f / ((red[4] + red[5]) + (red[6] + red[7]));
+        const float inv = 1.0f / red;
         const float g = 1.0f / (1.0f + expf(-gl));
-        const fv r = ((acc[0][lane] + acc[1][lane]) + (acc[2][lane] + acc[3][lane])) * inv * g;
+        fv r = acc[0][lane];
+#pragma unroll
+        for (int w = 1; w < W; w++) r += acc[w][lane];
+        r *= inv * g;
 #pragma unroll
         for (int v = 0; v < VPL; v++) {
-            out[lane * VPL + v] = r[v];
-            if (out16) out16[lane * VPL + v] = fw_bf16(r[v]);
+            out[row * HD + lane * VPL + v] = r[v];
+            if (out16) out16[row * HD + lane * VPL + v] = fw_bf16(r[v]);
         }
     }
-}
-
-template <int VPL>
-__global__ __launch_bounds__(256) void fw_attn_combine_kernel(const float * part, const float * gate, const int * st,
-                                                              int window, int nch_max, float * out, uint16_t * out16) {
-    constexpr int hd = 64 * VPL;
-    extern __shared__ float wts[];             /* per chunk: m_c, then e^(m_c - M); then l_c */
-    const int pos = st[1];
-    const int start = window > 0 && pos + 1 > window ? pos + 1 - window : 0;
-    const int nch = (pos + 1 - start + kAttnChunk - 1) / kAttnChunk;
-    const int h = blockIdx.x;
-    attn_combine_head<VPL>(part + (size_t) h * nch_max * (hd + 2), nch, gate[h], out + (size_t) h * hd,
-                           out16 ? out16 + (size_t) h * hd : nullptr, wts);
 }
 
 /* ---- a verify block: ntok <= 8 consecutive tokens at positions pos0 .. ----
@@ -485,80 +650,6 @@ __global__ __launch_bounds__(128) void fw_rope_kv_heads_kernel(float * qkv, int 
             kr[i + half] = r1;
         }
     }
-}
-
-/* Attention partials of token t = blockIdx.z (query rotated in qkv, every
- * key in the cache), as fw_attn_part_kernel otherwise. */
-template <int VPL>
-__global__ __launch_bounds__(256) void fw_attn_part_n_kernel(const float * qkv, int ldq, int kvd, const float * kc,
-                                                              const float * vc, int pos0, int window, int heads,
-                                                              int kv_heads, float scale, int nch_max, float * part) {
-    constexpr int hd = 64 * VPL, C = kAttnChunk;
-    typedef float fv __attribute__((ext_vector_type(VPL)));
-    const int t = blockIdx.z, pos = pos0 + t;
-    const int start = window > 0 && pos + 1 > window ? pos + 1 - window : 0;
-    const int n = pos + 1 - start;
-    const int chunk = blockIdx.x, kvh = blockIdx.y;
-    const int G = heads / kv_heads;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int j0 = chunk * C;
-    if (j0 >= n) return;
-    const int jn = min(C, n - j0);
-    const int h = kvh * G + wave;
-    const fv q = *(const fv *) (qkv + (size_t) t * ldq + (size_t) h * hd + lane * VPL);
-    const float * kb = kc + (size_t) (start + j0) * kvd + (size_t) kvh * hd + lane * VPL;
-    const float * vb = vc + (size_t) (start + j0) * kvd + (size_t) kvh * hd + lane * VPL;
-    fv kr[C], vr[C];
-#pragma unroll
-    for (int j = 0; j < C; j++) kr[j] = *(const fv *) (kb + (size_t) min(j, jn - 1) * kvd);
-#pragma unroll
-    for (int j = 0; j < C; j++) vr[j] = *(const fv *) (vb + (size_t) min(j, jn - 1) * kvd);
-    float sc[C];
-    float m = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < C; j++) {
-        float s = 0.0f;
-#pragma unroll
-        for (int v = 0; v < VPL; v++) s += q[v] * kr[j][v];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-        sc[j] = s * scale;
-        if (j < jn) m = fmaxf(m, sc[j]);
-    }
-    float l = 0.0f;
-    fv o = (fv) 0.0f;
-#pragma unroll
-    for (int j = 0; j < C; j++) {
-        /* rows past jn are padding that may hold anything (the row at pos
-         * before its store): skipped, not weighted by zero */
-        if (j < jn) {
-            const float e = expf(sc[j] - m);
-            l += e;
-            o += e * vr[j];
-        }
-    }
-    float * P = part + (((size_t) t * heads + h) * nch_max + chunk) * (hd + 2);
-    *(fv *) (P + lane * VPL) = o;
-    if (lane == 0) {
-        P[hd] = m;
-        P[hd + 1] = l;
-    }
-}
-
-/* The combine of token t = blockIdx.y: gates at gate + t * ldg, output row t. */
-template <int VPL>
-__global__ __launch_bounds__(256) void fw_attn_combine_n_kernel(const float * part, const float * gate, int ldg,
-                                                                int pos0, int window, int heads, int nch_max,
-                                                                float * out, uint16_t * out16) {
-    constexpr int hd = 64 * VPL;
-    extern __shared__ float wts[];
-    const int t = blockIdx.y, pos = pos0 + t;
-    const int start = window > 0 && pos + 1 > window ? pos + 1 - window : 0;
-    const int nch = (pos + 1 - start + kAttnChunk - 1) / kAttnChunk;
-    const int h = blockIdx.x;
-    const size_t ob = (size_t) t * heads * hd + (size_t) h * hd;
-    attn_combine_head<VPL>(part + ((size_t) t * heads + h) * nch_max * (hd + 2), nch, gate[(size_t) t * ldg + h],
-                           out + ob, out16 ? out16 + ob : nullptr, wts);
 }
 
 /* act = gelu(g) * u with torch's exact gelu, erf in f64 as model.rs:253-258
@@ -747,7 +838,6 @@ __global__ __launch_bounds__(256) void fw_attn_prompt_kernel(const float * qkv, 
  * V[4 g + ks][d], with the rows of O^T permuted (pa_d) so that d too runs in
  * groups of 4: the 16 lanes of a group read 256 contiguous bytes of a row. */
 constexpr int kPaTok = 16;     /* query tokens per workgroup */
-constexpr float kPaLag = 8.0f; /* how far a score may pass the reference maximum */
 
 /* head element contracted at k-step ks by lane group g in S^T = K Q^T */
 static __device__ __forceinline__ int pa_k(int ks, int g) { return 16 * (ks >> 2) + 4 * g + (ks & 3); }
@@ -991,9 +1081,9 @@ struct Model {
      * kernel (0: SPARKMV_SEPARATE_ACT=1 at creation; the same bits, slower) */
     int fuse_act = 1;
     int * st;                            /* token, position */
-    float * part;                        /* attention partials [heads][nch_max][head_dim + 2] */
+    float * part, * pml;                 /* attention partials [heads][nsplit][head_dim], [heads][nsplit][2] */
     float * rtab;                        /* rope tables [full, sliding][cos, sin][128] */
-    int nch_max;
+    int nsplit;                          /* kAttnSplits, or the tiles of a shorter cache */
     /* the recorded chain */
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -1009,7 +1099,7 @@ struct Model {
      * partials for verify blocks of up to 8 tokens */
     void * vmem = nullptr;
     int vcap = 0;
-    float * vh, * vxn, * vqkv, * vg, * vattn, * vmg, * vmu, * vact, * vpart;
+    float * vh, * vxn, * vqkv, * vg, * vattn, * vmg, * vmu, * vact, * vpart, * vpml;
     uint16_t * vxn16, * vattn16, * vact16;
     int * vtok;
     /* layer-input capture (model.rs:322-348, vq-model-gpu.cu:632-639):
@@ -1201,7 +1291,6 @@ void * sparkmv_model_create(const sparkmv_model_cfg * cfg) {
             return nullptr;
         }
     }
-    /* the combine keeps two floats per position chunk in LDS */
     const long nch_max = ((long) c.max_ctx + kAttnChunk - 1) / kAttnChunk;
     if (nch_max * 8 > 65536) { set_error("max_ctx %d is above %d", c.max_ctx, 8192 * kAttnChunk); return nullptr; }
     if (c.hidden > 8192) { set_error("hidden %d is above 8192", c.hidden); return nullptr; }
@@ -1219,7 +1308,8 @@ void * sparkmv_model_create(const sparkmv_model_cfg * cfg) {
     const size_t o_xn16 = take(c.hidden * 2), o_attn16 = take(qd * 2), o_act16 = take(c.intermediate * 2);
     const size_t o_kv = take((size_t) c.layers * c.max_ctx * kvd * 4 * 2);
     const size_t o_st = take(2 * sizeof(int));
-    const size_t o_part = take((size_t) c.heads * nch_max * (c.head_dim + 2) * 4);
+    const size_t nsplit = nch_max < kAttnSplits ? (size_t) nch_max : kAttnSplits;
+    const size_t o_part = take((size_t) c.heads * nsplit * c.head_dim * 4), o_pml = take((size_t) c.heads * nsplit * 8);
     const size_t o_rtab = take(512 * 4);
     const size_t n_pslot = (size_t) c.intermediate * kMaxCols;
     const size_t o_pslot = take(n_pslot * 8);
@@ -1252,8 +1342,9 @@ void * sparkmv_model_create(const sparkmv_model_cfg * cfg) {
     m->kv = (float *) (b + o_kv);
     m->st = (int *) (b + o_st);
     m->part = (float *) (b + o_part);
+    m->pml = (float *) (b + o_pml);
     m->rtab = (float *) (b + o_rtab);
-    m->nch_max = (int) nch_max;
+    m->nsplit = (int) nsplit;
     return m;
 }
 
@@ -1349,6 +1440,28 @@ int set_state(Model * m, uint32_t token, int pos, hipStream_t s) {
     return check_launch("state launch");
 }
 
+/* The split attention and its combine for one decode token (dec) or the
+ * block's A.N tokens, whose windows span at most `span` positions. */
+int attn_launch(const AttnArgs & A, int hd, int span, const float * gate, int ldg, float * out, uint16_t * out16,
+                bool dec, hipStream_t s) {
+    const int tiles = (span + kAttnChunk - 1) / kAttnChunk;
+    const dim3 grid((unsigned) (tiles < A.nsplit ? tiles : A.nsplit), (unsigned) A.kv_heads), b(256);
+    const bool two = A.N * (A.heads / A.kv_heads) > 16;
+#define FW_ATTN(H)                                                                                                   \
+    do {                                                                                                             \
+        if (dec) hipLaunchKernelGGL((fw_attn_split_kernel<H, 1, 1>), grid, b, 0, s, A);                              \
+        else if (two) hipLaunchKernelGGL((fw_attn_split_kernel<H, 2, 0>), grid, b, 0, s, A);                         \
+        else hipLaunchKernelGGL((fw_attn_split_kernel<H, 1, 0>), grid, b, 0, s, A);                                  \
+        hipLaunchKernelGGL(fw_attn_combine_kernel<H / 64>, dim3(A.heads, A.N), dim3(512), 0, s, A, dec ? 1 : 0, gate, \
+                           ldg, out, out16);                                                                         \
+    } while (0)
+    if (hd == 64) FW_ATTN(64);
+    else if (hd == 128) FW_ATTN(128);
+    else FW_ATTN(256);
+#undef FW_ATTN
+    return check_launch("attention launch");
+}
+
 /* Every launch of one token, reading token and position from m->st. */
 int chain(Model * m, float * logits, hipStream_t s) {
     const sparkmv_model_cfg & c = m->c;
@@ -1383,24 +1496,12 @@ int chain(Model * m, float * logits, hipStream_t s) {
          * the longest window this layer can see */
         const int pdim = rope_dim(hd, full ? c.rope_full_partial : c.rope_slide_partial);
         const float * rtab = m->rtab + (full ? 0 : 256);
-        const int window = full ? 0 : c.sliding_window;
         const int span = full || c.sliding_window > c.max_ctx ? c.max_ctx : c.sliding_window;
-        const int nch = (span + kAttnChunk - 1) / kAttnChunk;
-        const dim3 pg((unsigned) nch, (unsigned) c.kv_heads), pb((unsigned) (64 * (c.heads / c.kv_heads)));
-        const uint32_t wl = (uint32_t) (nch * 8);
-        uint16_t * a16 = b16 ? m->attn16 : nullptr;
-#define FW_ATTN(V)                                                                                                  \
-    do {                                                                                                            \
-        hipLaunchKernelGGL(fw_attn_part_kernel<V>, pg, pb, 0, s, m->qkv, qd, kvd, kc, vc, (const int *) m->st,        \
-                           window, c.heads, c.kv_heads, pdim, rtab, scale, m->nch_max, m->part);                    \
-        hipLaunchKernelGGL(fw_attn_combine_kernel<V>, dim3(c.heads), dim3(256), wl, s, m->part, m->g,               \
-                           (const int *) m->st, window, m->nch_max, m->attn, a16);                                  \
-    } while (0)
-        if (hd == 64) FW_ATTN(1);
-        else if (hd == 128) FW_ATTN(2);
-        else FW_ATTN(4);
-#undef FW_ATTN
-        if (check_launch("attention launch")) return -1;
+        AttnArgs at;
+        at.qkv = m->qkv; at.kc = kc; at.vc = vc; at.st = m->st; at.rtab = rtab; at.po = m->part; at.pml = m->pml;
+        at.ldq = qd + 2 * kvd; at.qd = qd; at.kvd = kvd; at.pos0 = 0; at.N = 1; at.window = full ? 0 : c.sliding_window;
+        at.heads = c.heads; at.kv_heads = c.kv_heads; at.pdim = pdim; at.nsplit = m->nsplit; at.scale = scale;
+        if (attn_launch(at, hd, span, m->g, 1, m->attn, b16 ? m->attn16 : nullptr, true, s)) return -1;
         if (gemv(*m, L.out, c.hidden, qd, b16 ? (const void *) m->attn16 : (const void *) m->attn, m->h, 1, s))
             return -1;
 
@@ -1442,7 +1543,8 @@ int alloc_block(Model * m, int cap) {
     const size_t o_g = take(N * (qd + 2 * kvd) * 4), o_attn = take(N * qd * 4), o_mg = take(N * c.intermediate * 4);
     const size_t o_mu = take(N * c.intermediate * 4), o_act = take(N * c.intermediate * 4);
     const size_t o_xn16 = take(N * c.hidden * 2), o_attn16 = take(N * qd * 2), o_act16 = take(N * c.intermediate * 2);
-    const size_t o_part = take((size_t) 8 * c.heads * (size_t) m->nch_max * (c.head_dim + 2) * 4);
+    const size_t o_part = take((size_t) 8 * c.heads * m->nsplit * c.head_dim * 4);
+    const size_t o_pml = take((size_t) 8 * c.heads * m->nsplit * 8);
     const size_t o_tok = take(N * sizeof(int));
     void * mem = nullptr;
     hipError_t e = hipMalloc(&mem, off);
@@ -1454,6 +1556,7 @@ int alloc_block(Model * m, int cap) {
     m->vh = (float *) (b + o_h); m->vxn = (float *) (b + o_xn); m->vqkv = (float *) (b + o_qkv);
     m->vg = (float *) (b + o_g); m->vattn = (float *) (b + o_attn); m->vmg = (float *) (b + o_mg);
     m->vmu = (float *) (b + o_mu); m->vact = (float *) (b + o_act); m->vpart = (float *) (b + o_part);
+    m->vpml = (float *) (b + o_pml);
     m->vxn16 = (uint16_t *) (b + o_xn16); m->vattn16 = (uint16_t *) (b + o_attn16);
     m->vact16 = (uint16_t *) (b + o_act16);
     m->vtok = (int *) (b + o_tok);
@@ -1523,24 +1626,13 @@ int block(Model * m, const uint32_t * tokens, int N, int pos, float * logits, hi
         const int pdim = rope_dim(hd, full ? c.rope_full_partial : c.rope_slide_partial);
         if (rope_kv_launch(m->vqkv, N, ldq, qd, kvd, c.heads, c.kv_heads, hd, pdim, (float) theta, pos, kc, vc, s))
             return -1;
-        const int window = full ? 0 : c.sliding_window;
-        const int last = pos + N - 1;
-        const int span = full || c.sliding_window > last + 1 ? last + 1 : c.sliding_window;
-        const int nch = (span + kAttnChunk - 1) / kAttnChunk;
-        const dim3 pg((unsigned) nch, (unsigned) c.kv_heads, (unsigned) N), pb((unsigned) (64 * (c.heads / c.kv_heads)));
-        uint16_t * a16 = b16 ? m->vattn16 : nullptr;
-#define FW_ATTN_N(V)                                                                                                \
-    do {                                                                                                            \
-        hipLaunchKernelGGL(fw_attn_part_n_kernel<V>, pg, pb, 0, s, m->vqkv, ldq, kvd, kc, vc, pos, window, c.heads,   \
-                           c.kv_heads, scale, m->nch_max, m->vpart);                                                \
-        hipLaunchKernelGGL(fw_attn_combine_n_kernel<V>, dim3(c.heads, N), dim3(256), (uint32_t) (nch * 8), s,       \
-                           m->vpart, m->vg, ldq, pos, window, c.heads, m->nch_max, m->vattn, a16);                  \
-    } while (0)
-        if (hd == 64) FW_ATTN_N(1);
-        else if (hd == 128) FW_ATTN_N(2);
-        else FW_ATTN_N(4);
-#undef FW_ATTN_N
-        if (check_launch("attention launch")) return -1;
+        AttnArgs at;
+        at.qkv = m->vqkv; at.kc = kc; at.vc = vc; at.st = nullptr; at.rtab = nullptr; at.po = m->vpart; at.pml = m->vpml;
+        at.ldq = ldq; at.qd = qd; at.kvd = kvd; at.pos0 = pos; at.N = N; at.window = full ? 0 : c.sliding_window;
+        at.heads = c.heads; at.kv_heads = c.kv_heads; at.pdim = pdim; at.nsplit = m->nsplit; at.scale = scale;
+        /* the block's positions: from the first token's window start to the last token */
+        const int span = full || pos + 1 < c.sliding_window ? pos + N : c.sliding_window + N - 1;
+        if (attn_launch(at, hd, span, m->vg, ldq, m->vattn, b16 ? m->vattn16 : nullptr, false, s)) return -1;
         if (gemv(*m, L.out, c.hidden, qd, b16 ? (const void *) m->vattn16 : (const void *) m->vattn, m->vh, 1, s, N,
                  c.hidden))
             return -1;

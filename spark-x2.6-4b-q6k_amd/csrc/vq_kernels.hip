@@ -29,6 +29,7 @@
 #include <hip/hip_fp16.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 
 namespace sparkmv {
@@ -140,7 +141,7 @@ __device__ __forceinline__ uint32_t bf16_rne(float f) {
 }
 
 template <int NST, int XF32, int EXT, int MSC, int MC, int XN = 0>
-__global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : 640) void vq_mfma_kernel(const FastArgs A) {
+__global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : MC == 2 && XF32 ? 512 : 640) void vq_mfma_kernel(const FastArgs A) {
     /* MSC > 0: a unit is exactly MSC macro steps, known at compile time, so
      * the whole unit runs as straight-line code and each step waits only for
      * its own index words (a loop would make the compiler wait for all of a
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : 640) void vq_mfma_kerne
      * squares in f64, 1 / sqrt rounded once to f32, (h * inv) * w in f32),
      * so the norm needs no launch of its own. */
     static_assert(!XN || (MC == 0 && MSC > 0 && !XF32), "the fused norm stages one bf16 column");
-    constexpr int XG = MC == 2 ? 1 : 0;
+    constexpr int XG = MC == 2 ? 1 + XF32 : 0;   /* 2: f32 x from global memory */
     constexpr int CK = MC == 3 ? 1 : 0;
     static_assert(!CK || (MSC > 0 && !XF32 && !XN), "chunk-split tiles run straight-line bf16 units");
     constexpr int D = MSC > 0 ? MSC : 8;
@@ -166,8 +167,9 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : 640) void vq_mfma_kerne
      * (one column: q+k+v+g 7.6 -> 7.4 us, down 9.7 -> 9.2 us against three;
      * one step ahead lost 0.2-0.8 us). The x-from-global kernels also carry
      * each step's x in the same loads and keep three below ten-step units
-     * (N = 8 down 14.8 -> 15.8 us with two). */
-    constexpr int kLook = (MSC >= 10 || !XG) ? 2 : 3;
+     * (N = 8 down 14.8 -> 15.8 us with two); with f32 x, whose steps hold
+     * twice the registers, two. */
+    constexpr int kLook = (MSC >= 10 || XG != 1) ? 2 : 3;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     /* cbb: bytes of one stage's codebook; cbs: their stride in LDS, a fixed
      * 32 KB for 12-bit indices (nc <= 4096), so the second stage's gathers
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : 640) void vq_mfma_kerne
     Words<NST, EXT, XG> w[D];
     /* XG: the lane's x run for its B column (part hp, activation column cn;
      * lanes past the parts read part 0 of column 0 and feed no output) */
-    const uint8_t * xgp = (const uint8_t *) A.x + ((size_t) (bval ? cn : 0) * A.ldx + 128 * msb + 32 * q) * 2;
+    const uint8_t * xgp = (const uint8_t *) A.x + ((size_t) (bval ? cn : 0) * A.ldx + 128 * msb + 32 * q) * (2 + 2 * XF32);
     auto ld = [&](Words<NST, EXT, XG> & W, int ms) {
         load_words<NST, EXT, XG>(W, rp, pp, xgp, ms < MS ? ms : MS - 1);
     };
@@ -348,10 +350,11 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : 640) void vq_mfma_kerne
                 for (int k = 0; k < KS; k++)
                     ((u4v *) (lds + s * cbs))[min(k * bd + tid, n16 - 1)] = cv[s][k];
         }
-        /* 8-column pieces of x per activation column; chunk-split tiles
+        /* 16-byte pieces of x per activation column; chunk-split tiles
          * stage the group's C * MS steps of each part, whose piece cc comes
          * from piece xsrc(cc) of the row */
-        const int xq = CK ? S * C * MS * 16 : A.cols >> 3, nx = XG ? 0 : ncol * xq;
+        constexpr int XP = XF32 ? 4 : 8;           /* columns per 16-byte piece */
+        const int xq = CK ? S * C * MS * 16 : A.cols / XP, nx = XG ? 0 : ncol * xq;
         auto xsrc = [&](int cc) {
             if constexpr (!CK) return cc;
             const int hh = cc / (C * MS * 16);
@@ -366,13 +369,26 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : 640) void vq_mfma_kerne
                 const int n = ci[k] / xq, cc = ci[k] - n * xq;
                 /* a slot wholly past x (uniform) would only repeat the last chunk */
                 if (base + k * bd < nx)
-                    xv[k] = *(const u4v *) ((const uint16_t *) A.x + (size_t) n * A.ldx + 8 * xsrc(cc));
+                    xv[k] = *(const u4v *) ((const uint8_t *) A.x + ((size_t) n * A.ldx + XP * xsrc(cc)) * (16 / XP));
             }
 #pragma unroll
             for (int k = 0; k < KXM; k++) {
                 if (base + k * bd >= nx) continue;
-                const int n = ci[k] / xq, e = 8 * (ci[k] - n * xq);
+                const int n = ci[k] / xq, e = XP * (ci[k] - n * xq);
                 uint8_t * dst = lx + n * A.xstride + 264 * (e >> 7) + 2 * (e & 127);
+                if constexpr (XF32) {
+                    h4 hi4, lo4;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float f = __uint_as_float(xv[k][j]);
+                        hi4[j] = (_Float16) f;
+                        lo4[j] = (_Float16) (f - (float) hi4[j]);
+                        xm = max(xm, xr_mag_f32w(xv[k][j]));
+                    }
+                    *(h4 *) dst = hi4;
+                    *(h4 *) (dst + ncol * A.xstride) = lo4;
+                    continue;
+                }
                 xr_acc_bf16x2(xm2, xv[k].x); xr_acc_bf16x2(xm2, xv[k].y);
                 xr_acc_bf16x2(xm2, xv[k].z); xr_acc_bf16x2(xm2, xv[k].w);
                 h4 lo4, hi4;
@@ -649,35 +665,42 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : 640) void vq_mfma_kerne
      * words and gains of the tile are already requested. */
     auto unit = [&](int tile) {
         const bool active = tile < t1;
-        f4 acc[NST];
+        constexpr int LOA = XF32 && MC ? 1 : 0;       /* the lo halves' sums apart */
+        constexpr int NA = LOA ? 2 * NST : NST;
+        f4 acc[NA];
 #pragma unroll
-        for (int s = 0; s < NST; s++) acc[s] = f4{0.f, 0.f, 0.f, 0.f};
-        /* XG: the largest bf16 |x| this lane converts in the unit, per half */
-        u16x2 xmx = {0, 0};
-        u16x2 * const xm = XG ? &xmx : nullptr;
+        for (int s = 0; s < NA; s++) acc[s] = f4{0.f, 0.f, 0.f, 0.f};
+        /* XG: the largest |x| this lane converts in the unit */
+        XMax xmx;
+        XMax * const xm = XG ? &xmx : nullptr;
         if (active) {
             if (MSC > 0) {
 #pragma unroll
                 for (int u = 0; u < D; u++) {
-                    mstep<NST, XF32, EXT, XG, 0>(w[u], cbs, xb + 264 * u, xbl + 264 * u, acc, 1.0f, xm);
+                    mstep<NST, XF32, EXT, XG, 0, LOA>(w[u], cbs, xb + 264 * u, xbl + 264 * u, acc, 1.0f, xm);
                     if (u + kLook < D) ld(w[u + kLook], u + kLook);
                     /* keep step u + kLook's loads here: left to itself the
                      * scheduler sinks them to just before their step, which
-                     * then waits a whole memory round trip. (XG units hold
-                     * 4 steps of x too: pinned, they would spill.) */
-                    if constexpr (!XG) __builtin_amdgcn_sched_barrier(0);
+                     * then waits a whole memory round trip. (Units of bf16 x from
+                     * global memory hold 4 steps of x too: pinned, they would
+                     * spill; those of f32 x spill unpinned.) */
+                    if constexpr (XG != 1) __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
                 for (int ms0 = 0; ms0 < MS; ms0 += D) {
 #pragma unroll
                     for (int u = 0; u < D; u++) {
                         if (ms0 + u < MS)
-                            mstep<NST, XF32, EXT, XG, 0>(w[u], cbs, xb + 264 * (ms0 + u), xbl + 264 * (ms0 + u), acc,
+                            mstep<NST, XF32, EXT, XG, 0, LOA>(w[u], cbs, xb + 264 * (ms0 + u), xbl + 264 * (ms0 + u), acc,
                                                       1.0f, xm);
                         if (MS > D) ld(w[u], ms0 + u + D);
                     }
                 }
             }
+        }
+        if constexpr (LOA) {
+#pragma unroll
+            for (int s = 0; s < NST; s++) acc[s] += acc[NST + s];
         }
         /* the factor 2^uk that the unit's sums carry back */
         int uk = xk;
@@ -702,36 +725,41 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : 640) void vq_mfma_kerne
 #pragma unroll
                     for (int i = 0; i < 4; i++) bad = bad || !__builtin_isfinite(acc[s][i]);
                 /* as f32 bits; a non-finite maximum is never small */
-                uint32_t m = xr_col_max((uint32_t) max(xmx[0], xmx[1]) << 16);
+                uint32_t m = xr_col_max(XF32 ? xmx.f32() : xmx.bf16());
                 const bool small = m != 0u && m < kXrLow;
                 if (__builtin_amdgcn_ballot_w64(bad || small)) {
-                    if (__builtin_amdgcn_ballot_w64(bad)) {
+                    if (XF32 || __builtin_amdgcn_ballot_w64(bad)) {
                         typedef uint32_t u4x __attribute__((ext_vector_type(4)));
                         m = 0;
 #pragma unroll 1
                         for (int u = 0; u < MS; u++) {
 #pragma unroll
-                            for (int k = 0; k < 4; k++) {
-                                const u4x v = ((const u4x *) (xgp + 256 * u))[k];
+                            for (int k = 0; k < 4 * XG; k++) {
+                                const u4x v = ((const u4x *) (xgp + 256 * XG * u))[k];
 #pragma unroll
                                 for (int h = 0; h < 4; h++)
-                                    m = max(m, max(xr_fin((v[h] << 16) & 0x7fffffffu), xr_fin(v[h] & 0x7fff0000u)));
+                                    m = max(m, XF32 ? xr_fin(xr_mag_f32w(v[h]))
+                                                    : max(xr_fin((v[h] << 16) & 0x7fffffffu), xr_fin(v[h] & 0x7fff0000u)));
                             }
                         }
                         m = xr_col_max(m);   /* the column's largest finite |x| in the unit */
                     }
-                    /* 2^-uk must be a normal f32: bf16 x below 2^-126 is
+                    /* 2^-uk must be a normal f32: x below 2^-126 is
                      * brought up only as far as 2^126 takes it */
                     uk = max(xr_shift_of(m), -126);
                     if (__builtin_amdgcn_ballot_w64(uk != 0)) {
                         const float sc = __uint_as_float((uint32_t) (127 - uk) << 23);
 #pragma unroll
-                        for (int s = 0; s < NST; s++) acc[s] = f4{0.f, 0.f, 0.f, 0.f};
+                        for (int s = 0; s < NA; s++) acc[s] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
                         for (int u = 0; u < MS; u++) {
                             Words<NST, EXT, XG> W1;
                             load_words<NST, EXT, XG>(W1, rp, pp, xgp, u);
-                            mstep<NST, XF32, EXT, XG, 1>(W1, cbs, xb, xbl, acc, sc);
+                            mstep<NST, XF32, EXT, XG, 1, LOA>(W1, cbs, xb, xbl, acc, sc);
+                        }
+                        if constexpr (LOA) {
+#pragma unroll
+                            for (int s = 0; s < NST; s++) acc[s] += acc[NST + s];
                         }
                     }
                 }
@@ -1107,6 +1135,7 @@ struct FastShape {
     int xg;   /* several columns with x read from global memory (no x in LDS) */
     int sk;   /* shared tiles: W (tile, chunk) units per workgroup */
     int ck;   /* chunk-split tiles: groups of C chunks per tile (0: none) */
+    int sf;   /* several f32 columns staged in LDS, straight-line units */
 };
 
 /* LDS bytes per activation column: 264 bytes per 128 columns (256 of f16
@@ -1124,28 +1153,34 @@ static size_t fast_lds(const VqCall & c, int nst, int S, int W, int xg = 0) {
            (size_t) W * kRedStride * 4 + kXrBytes;
 }
 
-/* Several bf16 columns with x read from global memory: each lane loads its
- * 32 activations of a step (64 bytes, 16-byte aligned rows) with the step's
- * index words, so nothing but codebooks sits in LDS and no column count
- * splits K. Taken when x is at least 48 KB (N = 8 at 4096 and 10240
- * columns: staging it cost more than its loads, measured); smaller x is
- * staged in LDS. Straight-line units only (a ring would hold 8 steps of x
- * per lane), at most 10 waves (the registers of 4 steps in flight), and
- * enough threads to stage the codebooks in 5 chunks each. Shape: fewest
+/* Several columns with x read from global memory: each lane loads its 32
+ * activations of a step (16-byte aligned rows) with the step's index words,
+ * so nothing but codebooks sits in LDS and no column count splits K. bf16 x
+ * takes it from 48 KB (N = 8 at 4096 and 10240 columns: staging it cost more
+ * than its loads, measured); smaller bf16 x is staged in LDS. f32 x
+ * takes it where hi + lo f16 of every column does not fit LDS in one K range
+ * (fast_shape_f32 below takes the rest): a launch per K range in the ring
+ * form made five columns of down three launches of 94.6 us in all; 19.3 here.
+ * Straight-line units only (a ring would hold 8 steps of x per lane), at most
+ * 10 waves (the registers of 4 steps in flight; 8 for f32 x, whose steps hold
+ * twice as many), and enough threads to stage the codebooks in 5 chunks each.
+ * Shape: fewest
  * rounds of workgroups over the CUs, then the shortest unit. */
 static int fast_shape_xg(const VqCall & c, int nst, FastShape & sh) {
-    if (c.ncol < 2 || c.xf32 || c.nc % 2 || ((uintptr_t) c.x & 15u) || c.ldx % 8) return -1;
-    if ((long) c.ncol * c.cols < 24576) return -1;
+    if (c.ncol < 2 || c.nc % 2 || ((uintptr_t) c.x & 15u) || c.ldx % (c.xf32 ? 4 : 8)) return -1;
+    if (!c.xf32 && (long) c.ncol * c.cols < 24576) return -1;
     const int M = c.cols / 128, G = cu_count(), n16 = c.nc * 8 / 16;
+    /* f32 x: eight waves, for the registers of three steps of x */
+    const int wmax = c.xf32 ? 8 : 10;
     long best = -1;
     for (int s = 1; s <= 16; s *= 2) {
         if (s * c.ncol > 16 || M % s) continue;
         const int MP = M / s;
-        for (int cc = 1; cc <= 10; cc++) {
+        for (int cc = 1; cc <= wmax; cc++) {
             if (MP % cc) continue;
             const int ms = MP / cc;
-            if (ms != 2 && ms != 4 && ms != 5 && ms != 8 && (ms != 10 || c.nc > 4096)) continue;
-            for (int tt = 1; tt * cc <= 10; tt++) {
+            if (ms != 2 && ms != 4 && ms != 5 && (ms != 8 || c.xf32) && (ms != 10 || c.nc > 4096)) continue;
+            for (int tt = 1; tt * cc <= wmax; tt++) {
                 if (5 * 64 * tt * cc < n16) continue;
                 long nwg = 0;
                 for (int m = 0; m < c.nmat; m++) nwg += ((c.mats[m].rows * (long) s + 15) / 16 + tt - 1) / tt;
@@ -1169,7 +1204,7 @@ static int fast_shape_xg(const VqCall & c, int nst, FastShape & sh) {
      * not pay for their own staging (N = 8 over 4096 columns: 2-step units
      * measured slower than whole tiles on 160 CUs). */
     if (c.kslot && c.nmat == 1 && (long) c.mats[0].rows * c.ncol <= c.kslot_cap && 5 * sh.nwg < 4 * G) {
-        const int W = 10;
+        const int W = wmax;
         int bn = 0, bms = 0;
         for (int s = 1; s <= 16; s *= 2) {
             if (s * c.ncol > 16 || M % s) continue;
@@ -1178,7 +1213,7 @@ static int fast_shape_xg(const VqCall & c, int nst, FastShape & sh) {
             for (int cc = 2; cc <= W; cc++) {
                 if (MP % cc) continue;
                 const int ms = MP / cc;
-                if (ms != 4 && ms != 5 && ms != 8 && (ms != 10 || c.nc > 4096)) continue;
+                if (ms != 4 && ms != 5 && (ms != 8 || c.xf32) && (ms != 10 || c.nc > 4096)) continue;
                 if (5 * 64 * W < n16) continue;
                 const long nwg = (tiles * cc + W - 1) / W;
                 const size_t lds = fast_lds(c, nst, s, W, 1);
@@ -1242,14 +1277,62 @@ static int fast_shape_ck(const VqCall & c, int nst, FastShape & sh) {
     return best < 0 ? -1 : 0;
 }
 
+/* The unit lengths with a straight-line one-column kernel (launch_ms and
+ * launch_ms_norm below). */
+static int straight_ms(int MS, int ext, int norm) {
+    switch (MS) {
+        case 1: case 2: case 4: case 5: case 8: return 1;
+        case 3: case 6: return !norm;
+        case 10: return !ext;
+        default: return 0;
+    }
+}
+
+/* Several f32 columns staged in LDS as hi + lo f16, straight-line units:
+ * taken where they fit beside the codebooks in one K range, since a value is
+ * then split once per workgroup and not once per tile (N = 8 gate+up: 44.2 us
+ * with x from global memory, 31.6 in the ring form, 18.9 here). The search is
+ * the staged bf16 one over the unit lengths with a kernel. */
+static int fast_shape_f32(const VqCall & c, int nst, FastShape & sh) {
+    if (!c.xf32 || c.ncol < 2 || c.nc % 2 || ((uintptr_t) c.x & 15u) || c.ldx % 4) return -1;
+    const int M = c.cols / 128, G = cu_count(), n16 = c.nc * 8 / 16;
+    long best = -1;
+    for (int s = 1; s <= 16; s *= 2) {
+        if (s * c.ncol > 16 || M % s) continue;
+        const int MP = M / s;
+        for (int cc = 1; cc <= 16; cc++) {
+            if (MP % cc) continue;
+            const int ms = MP / cc;
+            if (ms != 2 && ms != 4 && ms != 5 && ms != 8 && (ms != 10 || c.nc > 4096)) continue;
+            for (int tt = 1; tt * cc <= 16; tt++) {
+                if (5 * 64 * tt * cc < n16) continue;
+                long nwg = 0;
+                for (int m = 0; m < c.nmat; m++) nwg += ((c.mats[m].rows * (long) s + 15) / 16 + tt - 1) / tt;
+                const size_t lds = fast_lds(c, nst, s, tt * cc);
+                if (lds > (size_t) kLdsMax) continue;
+                const long cost = (nwg + G - 1) / G * (8 + ms + cc - 1) * 64 + tt * cc;
+                if (best < 0 || cost < best) {
+                    best = cost;
+                    sh.S = s; sh.C = cc; sh.T = tt; sh.W = tt * cc; sh.nwg = (int) nwg; sh.lds = lds;
+                    sh.xg = 0; sh.sk = 0; sh.sf = 1;
+                }
+            }
+        }
+    }
+    return best < 0 ? -1 : 0;
+}
+
 static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
     sh.ck = 0;
+    sh.sf = 0;
+    if (fast_shape_f32(c, nst, sh) == 0) return 0;
     if (kFastXg && fast_shape_xg(c, nst, sh) == 0) {
         /* where x from global memory would take shared tiles (whole tiles
          * leave CUs idle), chunk-split tiles instead: N = 8 down 14.7 ->
          * 13.1-13.6 us, measured; for o (whole tiles on 160 CUs) they gave
          * -0.45 and +0.2 us on two boxes, and o keeps its shape */
         FastShape ck;
+        ck.sf = 0;
         if (sh.sk && fast_shape_ck(c, nst, ck) == 0) sh = ck;
         return 0;
     }
@@ -1273,8 +1356,13 @@ static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
     }
     if (!S) { set_error("no MFMA part split fits %d columns and %d macro steps", c.ncol, M); return -1; }
     const long tiles = tiles_for(S);
+    const int n16 = c.nc * 8 / 16;                 /* 16-byte chunks of a codebook */
+    /* one column whose unit of all of a part's steps has a straight-line
+     * kernel does not split it into chunks (which run the ring form) */
+    const int straight1 = c.ncol == 1 && straight_ms(M / S, c.nc > 4096, 0) && c.nc % 2 == 0 && n16 <= 3200 &&
+                          c.cols <= 10240 && !((uintptr_t) c.x & 15u);
     int C = 1;
-    if (tiles < want) {
+    if (tiles < want && !straight1) {
         const int MP = M / S;
         for (int cc = 2; cc <= 10; cc++) {
             if (MP % cc || MP / cc < 2) continue;
@@ -1287,6 +1375,14 @@ static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
     if (T * C > 10) T = 10 / C > 0 ? 10 / C : 1;
     if (T * C > 10) { C = 10; T = 1; }
     sh.S = S; sh.C = C; sh.T = T; sh.W = T * C;
+    if (c.ncol == 1) {
+        /* Short matrices leave a workgroup one to six waves, too few to stage
+         * the codebooks in one pass of five chunks per thread and stage (and
+         * x in two), which the straight-line kernels ask for and the ring
+         * form is slow without: waves past the tiles stage and then end. One
+         * f32 column of 1024 x 2560 22.0 -> 8.9 us. */
+        sh.W = std::max(sh.W, std::max(std::min(10, (n16 + 319) / 320), std::min(10, (c.cols + 1023) / 1024)));
+    }
     sh.nwg = 0;
     for (int m = 0; m < c.nmat; m++) sh.nwg += (int) (((c.mats[m].rows * (long) S + 15) / 16 + T - 1) / T);
     sh.lds = fast_lds(c, nst, S, sh.W);
@@ -1301,7 +1397,6 @@ static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
         /* 16 waves only in the multi-column kernels (bf16 x, even codebook,
          * 16-byte aligned x rows, at least 5 codebook chunks' worth of threads) */
         const int mc_ok = !c.xf32 && c.nc % 2 == 0 && !((uintptr_t) c.x & 15u) && c.ldx % 8 == 0;
-        const int n16 = c.nc * 8 / 16;
         long best = -1;
         for (int s = 1; s <= 16; s *= 2) {
             if (s * c.ncol > 16 || M % s) continue;
@@ -1333,9 +1428,9 @@ static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
     return 0;
 }
 
-/* Units of 1-6, 8 or 10 macro steps (the trunk's shapes give 2, 5 and 10)
- * run the straight-line kernel for bf16 x; any other length, and f32 x, the
- * ring kernel. Thirteen-bit indices hold plane bytes too, so their
+/* Units of 1-6, 8 or 10 macro steps (the trunk's shapes give 2, 5 and 10;
+ * several columns 2, 4, 5, 8 or 10) run the straight-line kernels; any other
+ * length the ring kernel. Thirteen-bit indices hold plane bytes too, so their
  * straight-line units stop at 8 steps (10 would spill). */
 /* The one-column straight-line kernels that stage rms_norm(h) themselves. */
 template <int NST, int EXT, int XN>
@@ -1429,12 +1524,44 @@ static int launch_ms(const FastArgs & A, int MS, int mc, int grid, int threads, 
         /* f32 x, one column: the trunk's unit lengths run straight-line too
          * (x as hi + lo f16 in LDS, two MFMAs per step) */
         switch (MS) {
+            case 1: return launch_fast_t<NST, 1, EXT, 1>(A, grid, threads, lds, s);
             case 2: return launch_fast_t<NST, 1, EXT, 2>(A, grid, threads, lds, s);
+            case 3: return launch_fast_t<NST, 1, EXT, 3>(A, grid, threads, lds, s);
+            case 4: return launch_fast_t<NST, 1, EXT, 4>(A, grid, threads, lds, s);
             case 5: return launch_fast_t<NST, 1, EXT, 5>(A, grid, threads, lds, s);
+            case 6: return launch_fast_t<NST, 1, EXT, 6>(A, grid, threads, lds, s);
             case 8: return launch_fast_t<NST, 1, EXT, 8>(A, grid, threads, lds, s);
             case 10: if (!EXT) return launch_fast_t<NST, 1, EXT, EXT ? 0 : 10>(A, grid, threads, lds, s); break;
             default: break;
         }
+    } else if (mc == 1) {
+        /* several f32 columns staged in LDS: the search kept to these unit
+         * lengths */
+        switch (MS) {
+            case 2: return launch_fast_t<NST, 1, EXT, 2, 1>(A, grid, threads, lds, s);
+            case 4: return launch_fast_t<NST, 1, EXT, 4, 1>(A, grid, threads, lds, s);
+            case 5: return launch_fast_t<NST, 1, EXT, 5, 1>(A, grid, threads, lds, s);
+            case 8: return launch_fast_t<NST, 1, EXT, 8, 1>(A, grid, threads, lds, s);
+            case 10:
+                if constexpr (!EXT) return launch_fast_t<NST, 1, EXT, 10, 1>(A, grid, threads, lds, s);
+                break;
+            default: break;
+        }
+        set_error("no staged f32 kernel for units of %d macro steps", MS);
+        return -1;
+    } else {
+        /* several f32 columns: x from global memory */
+        switch (MS) {
+            case 2: return launch_fast_t<NST, 1, EXT, 2, 2>(A, grid, threads, lds, s);
+            case 4: return launch_fast_t<NST, 1, EXT, 4, 2>(A, grid, threads, lds, s);
+            case 5: return launch_fast_t<NST, 1, EXT, 5, 2>(A, grid, threads, lds, s);
+            case 10:
+                if constexpr (!EXT) return launch_fast_t<NST, 1, EXT, 10, 2>(A, grid, threads, lds, s);
+                break;
+            default: break;
+        }
+        set_error("no x-from-global kernel for units of %d macro steps", MS);
+        return -1;
     }
     return launch_fast_t<NST, XF32, EXT, 0>(A, grid, threads, lds, s);
 }
@@ -1450,17 +1577,6 @@ struct FastNorm {
 /* nrm: stage bf16(rms_norm(x) * w) from the f32 residual x (one column, the
  * whole row in one launch, a one-column straight-line shape); returns 1
  * without launching when the call's shape has no such kernel. */
-/* The unit lengths with a straight-line one-column kernel (launch_ms and
- * launch_ms_norm below). */
-static int straight_ms(int MS, int ext, int norm) {
-    switch (MS) {
-        case 1: case 2: case 4: case 5: case 8: return 1;
-        case 3: case 6: return !norm;
-        case 10: return !ext;
-        default: return 0;
-    }
-}
-
 static int launch_fast_part(const VqCall & c, int st0, int nst, int accumulate, int k0, int mk,
                             const FastNorm * nrm = nullptr, const VqPair * pair = nullptr) {
     const Layout L0 = make_layout(c.dim, c.nc, c.mats[0].rows, c.cols, 1);
@@ -1518,12 +1634,13 @@ static int launch_fast_part(const VqCall & c, int st0, int nst, int accumulate, 
      * column of f32 x. One column is staged in one branch-free pass and
      * reduced within a wave: 16-byte aligned x of at most 16 * threads
      * values, one wave per tile, at most 5 codebook chunks per thread and
-     * stage. Several bf16 columns are staged by loops before the index words
+     * stage. Several columns are staged by loops before the index words
      * are requested. */
     const int n16 = c.nc * 8 / 16;
     const int one_col = sh.C == 1 && !((uintptr_t) A.x & 15u) && n16 <= 5 * threads && part.cols <= 16 * threads;
-    const int multi_col = c.ncol > 1 && !((uintptr_t) A.x & 15u) && c.ldx % 8 == 0 && n16 <= 5 * threads;
-    const int straight = (!c.xf32 || c.ncol == 1) && c.nc % 2 == 0 && (c.ncol > 1 ? multi_col : one_col);
+    const int multi_col =
+        c.ncol > 1 && !((uintptr_t) A.x & 15u) && c.ldx % (c.xf32 ? 4 : 8) == 0 && n16 <= 5 * threads;
+    const int straight = (!c.xf32 || c.ncol == 1 || sh.sf) && c.nc % 2 == 0 && (c.ncol > 1 ? multi_col : one_col);
     const int MS = sh.xg ? A.M / sh.S / sh.C : sh.ck ? A.M / sh.S / sh.C / sh.ck : straight ? A.M / sh.S / sh.C : 0;
     /* the multi-column kernels: x from global memory (2) or staged in LDS (1;
      * MS without its own instantiation runs their ring form); any other

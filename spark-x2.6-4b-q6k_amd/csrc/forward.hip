@@ -43,6 +43,8 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <atomic>
+
 #include <map>
 #include <vector>
 
@@ -848,7 +850,8 @@ __global__ __launch_bounds__(256) void fw_attn_prompt_mfma_kernel(const float * 
                                                                    const float * kc, const float * vc,
                                                                    const float * gate, int ldg, int pos0, int N,
                                                                    int window, int heads, int kv_heads, float scale,
-                                                                   float * out, uint16_t * out16) {
+                                                                   float * out, uint16_t * out16,
+                                                                   const uint32_t * redo, int nredo) {
     typedef float f4v __attribute__((ext_vector_type(4)));
     /* the merge after the loop: outputs handed between waves, 3 x 4 blocks
      * of 64 x 4 floats per wave, and the maximum and sum per token of each;
@@ -858,6 +861,13 @@ __global__ __launch_bounds__(256) void fw_attn_prompt_mfma_kernel(const float * 
     const int h = blockIdx.x, t0 = ((int) gridDim.y - 1 - (int) blockIdx.y) * kPaTok;
     const int kvh = h / (heads / kv_heads);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, c = lane & 15;
+    if (redo) {
+        /* after the split kernel below: only the blocks that it could not do */
+        const int nb = ((int) gridDim.y + 1) / 2;   /* its blocks are two of these */
+        uint32_t any = 0;
+        for (int z = 0; z < nredo; z++) any |= redo[((size_t) z * nb + t0 / (2 * kPaTok)) * kv_heads + kvh];
+        if (!any) return;   /* uniform */
+    }
     /* this lane's token (column c); tokens past N compute a copy of the last
      * one and store nothing */
     const int tv = min(t0 + c, N - 1), pos_t = pos0 + tv;
@@ -1052,6 +1062,392 @@ __global__ __launch_bounds__(256) void fw_attn_prompt_mfma_kernel(const float * 
     } else {
 #pragma unroll
         for (int i = 0; i < 4; i++) *(f4v *) (out + ob + 4 * i) = r[i];
+    }
+}
+
+/* Prompt attention over long spans, for 256-element heads in groups of four
+ * query heads per kv head: the products on the f16 matrix cores, f32 in
+ * value. Every f32 operand is brought to the top of f16's range by a power of
+ * two (exact: per token for q, per position for k, per four positions for v,
+ * whose weights take the quotient to the tile's largest) and split into two
+ * f16 halves, hi + lo = x to 2^-23 of x; hi hi, hi lo and lo hi are taken (lo
+ * lo is below 2^-24). Three f16 products run in 3/16 of the f32 products'
+ * matrix-core time. Sums stay f32: hi hi and the small products of the scores
+ * have an accumulator each, and the outputs of 32 positions are summed apart,
+ * small products first, then added to the running output: it rounds once per
+ * 32 positions (the f32 kernel above, every 4). Distance of f32 logits from
+ * the 64-bit ones, both within 0.5 % of each other: 1.34e-6 (12 tokens at
+ * 3000), 2.03e-6 (16 at 16000).
+ *
+ * One workgroup per (kv head, 32 tokens, span split): of its eight waves,
+ * wave w is query head w % 4 of the group and tokens 16 (w / 4) .. against all
+ * of the workgroup's K and V, so a position's rows are read, split and put
+ * into LDS once for 128 columns (the f32 kernel reads them per head and 16
+ * tokens). Positions go 32 at a time. The query halves and the outputs (64
+ * registers each) stay in registers; K is converted while the outputs' MFMAs
+ * run, V while the scores' do, each requested a phase earlier.
+ *
+ * 512 tokens at 16384, 16 heads: 592 us, 1378 in the f32 kernel (101 TFLOP/s
+ * of f32 products; 236 here). What bounds it is the conversions' and
+ * softmax's VALU work and the two barriers per tile (MFMAs are busy a quarter
+ * of the time). Nothing may spill here: a wave's loads return in order, so a
+ * reload in the loop waits for the K and V requests before it (59 spilled
+ * registers: 1400 us). Three bf16 planes and six products need no scales but
+ * spilled, at 1390 us.
+ *
+ * Layouts (16x16x32: lane l = 16 g + c holds A[c][8 g + j], B[8 g + j][c],
+ * D[4 g + i][c]): scores are positions x tokens, so a lane's 8 weights are of
+ * its own token, and the output product takes weight j as it lies: position
+ * 16 (j / 4) + 4 g + j % 4, with V stored to match. Output block b, row r is
+ * head element 16 r + b.
+ *
+ * A workgroup that meets an infinity or NaN says so in redo [split][token
+ * block][kv head], and the f32 kernel above then does those blocks again. */
+constexpr int kPsTok = 32;                          /* tokens per workgroup, positions per tile */
+constexpr int kPsPlane = 16384;                     /* LDS bytes of one half of a tile */
+constexpr int kPsLds = 4 * kPsPlane + 256;          /* K and V halves, scales, the waves' flags */
+constexpr int kPsMaxSplit = 8;
+
+typedef uint32_t ps_u4 __attribute__((ext_vector_type(4)));
+typedef _Float16 ps_h8 __attribute__((ext_vector_type(8)));
+
+/* f[0 .. 7] * sc as two halves of eight f16 */
+static __device__ __forceinline__ void ps_split(const float * f, float sc, ps_h8 * pl) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const float x = f[j] * sc;
+        pl[0][j] = (_Float16) x;
+        pl[1][j] = (_Float16) (x - (float) pl[0][j]);
+    }
+}
+
+/* The largest of m over the 16 lanes of a row, in every lane */
+static __device__ __forceinline__ uint32_t ps_max16(uint32_t m) {
+    m = max(m, (uint32_t) __builtin_amdgcn_update_dpp(0, (int) m, 0xB1, 0xf, 0xf, false));    /* lane ^ 1 */
+    m = max(m, (uint32_t) __builtin_amdgcn_update_dpp(0, (int) m, 0x4E, 0xf, 0xf, false));    /* lane ^ 2 */
+    m = max(m, (uint32_t) __builtin_amdgcn_update_dpp(0, (int) m, 0x141, 0xf, 0xf, false));   /* mirrored in 8 */
+    return max(m, (uint32_t) __builtin_amdgcn_update_dpp(0, (int) m, 0x140, 0xf, 0xf, false)); /* in 16 */
+}
+
+/* The power of two that brings the largest magnitude (f32 bits) to [2^14,
+ * 2^15), and its inverse */
+static __device__ __forceinline__ float ps_scale(uint32_t mag, float & inv) {
+    const uint32_t f = mag == 0u ? 127u : min(268u - min(mag >> 23, 254u), 253u);
+    inv = __uint_as_float((254u - f) << 23);
+    return __uint_as_float(f << 23);
+}
+
+typedef float ps_f4 __attribute__((ext_vector_type(4)));
+
+static __device__ __forceinline__ ps_f4 ps_mfma(ps_h8 a, ps_h8 b, ps_f4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+__global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float * qkv, int ldq, int kvd,
+                                                                    const float * kc, const float * vc, int pos0, int N,
+                                                                    int window, int heads, float scale, float * po,
+                                                                    float * pml, uint32_t * redo) {
+    typedef ps_f4 f4v;
+    typedef _Float16 h4v __attribute__((ext_vector_type(4)));
+    extern __shared__ __attribute__((aligned(16))) uint8_t ps_lds[];
+    float * kinv = (float *) (ps_lds + 4 * kPsPlane);          /* K's inverse scale per position */
+    float * vinv = kinv + 32;                                  /* V's per four positions 16 pb + 4 g .., at [2 g + pb] */
+    uint32_t * flags = (uint32_t *) (vinv + 8);                /* per wave, at the end */
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, c = lane & 15;
+    /* the blocks with the longest causal range first */
+    const int kvh = blockIdx.z, t0 = ((int) gridDim.y - 1 - (int) blockIdx.y) * kPsTok, h = 4 * kvh + (wave & 3);
+    const int tk = t0 + 16 * (wave >> 2) + c;
+    const int tv = min(tk, N - 1), pos_t = pos0 + tv;
+    const int start_t = window > 0 && pos_t + 1 > window ? pos_t + 1 - window : 0;
+    const int pfirst = window > 0 && pos0 + t0 + 1 > window ? pos0 + t0 + 1 - window : 0;
+    const int plast = pos0 + min(t0 + kPsTok - 1, N - 1);
+    const int nt = (plast - pfirst) / 32 + 1, nz = gridDim.x, z = blockIdx.x;
+    const int ta = (int) ((long) nt * z / nz), tb = (int) ((long) nt * (z + 1) / nz);
+    const float * kb = kc + (size_t) kvh * 256, * vb = vc + (size_t) kvh * 256;
+    const float * qrow = qkv + (size_t) tv * ldq + (size_t) h * 256;
+
+    /* K: piece i is position 16 i + tid / 32, elements 8 kg .. + 7; positions
+     * past plast repeat it and are masked */
+    const int kg = tid & 31, kp = tid >> 5;
+    f4v kr[4], vr[4];
+    auto load_k = [&](int p0) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const f4v * r = (const f4v *) (kb + (size_t) min(p0 + 16 * i + kp, plast) * kvd + 8 * kg);
+            kr[2 * i] = r[0];
+            kr[2 * i + 1] = r[1];
+        }
+    };
+    float ksc[2];
+    bool bad = false;   /* an infinity or NaN */
+    /* the pieces' scales, from their positions' largest magnitudes (32 lanes) */
+    auto scale_k = [&]() {
+        uint32_t all = 0;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            uint32_t m = 0;
+#pragma unroll
+            for (int j = 0; j < 8; j++) m = max(m, __float_as_uint(kr[2 * i + (j >> 2)][j & 3]) & 0x7fffffffu);
+            m = ps_max16(m);
+            m = max(m, (uint32_t) __shfl_xor((int) m, 16, 64));
+            all = max(all, m);
+            float inv;
+            ksc[i] = ps_scale(m, inv);
+            if (kg == 0) kinv[16 * i + kp] = inv;
+        }
+        bad |= all >= 0x7f800000u;
+    };
+    /* a half's 16-byte pieces by (element group, position), the positions of
+     * a group permuted so that neither side meets bank conflicts */
+    auto store_k = [&](int i) {
+        float f[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) f[j] = kr[2 * i + (j >> 2)][j & 3];
+        ps_h8 pl[2];
+        ps_split(f, ksc[i], pl);
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+            *(ps_h8 *) (ps_lds + p * kPsPlane + kg * 512 + 16 * ((16 * i + kp) ^ (kg & 15))) = pl[p];
+    };
+    /* V: wave 2 vg + pb takes positions 16 pb + 4 vg .. + 3, elements 4 lane .. + 3 */
+    const int vg = wave >> 1, vp = wave & 1;
+    auto load_v = [&](int p0) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            vr[j] = *(const f4v *) (vb + (size_t) min(p0 + 16 * vp + 4 * vg + j, plast) * kvd + 4 * lane);
+    };
+    float vsc = 1.0f;
+    auto scale_v = [&]() {
+        uint32_t m = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) m = max(m, __float_as_uint(vr[j][e]) & 0x7fffffffu);
+        m = ps_max16(m);
+        m = max(m, (uint32_t) __shfl_xor((int) m, 16, 64));
+        m = max(m, (uint32_t) __shfl_xor((int) m, 32, 64));
+        float inv;
+        vsc = ps_scale(m, inv);
+        if (lane == 0) vinv[wave] = inv;
+        bad |= m >= 0x7f800000u;
+    };
+    /* element 4 lane + e is row lane / 4 of block 4 (lane % 4) + e */
+    auto store_v = [&](int e) {
+        h4v hi, lo;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float x = vr[j][e] * vsc;
+            hi[j] = (_Float16) x;
+            lo[j] = (_Float16) (x - (float) hi[j]);
+        }
+        uint8_t * d = ps_lds + 2 * kPsPlane + (4 * (lane & 3) + e) * 1024 + vg * 256 + (lane >> 2) * 16 + vp * 8;
+        *(h4v *) d = hi;
+        *(h4v *) (d + kPsPlane) = lo;
+    };
+
+    if (ta < tb) {
+        load_k(pfirst + 32 * ta);
+        load_v(pfirst + 32 * ta);
+    }
+    /* the token's query: halves of the row's 8 steps, the row's scale over the
+     * four lanes that hold it */
+    ps_h8 q[8][2];
+    float qinv;
+    {
+        f4v qf[16];
+        uint32_t mx = 0;
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++) {
+            qf[ks] = *(const f4v *) (qrow + 32 * (ks >> 1) + 8 * g + 4 * (ks & 1));
+#pragma unroll
+            for (int j = 0; j < 4; j++) mx = max(mx, __float_as_uint(qf[ks][j]) & 0x7fffffffu);
+        }
+        mx = max(mx, (uint32_t) __shfl_xor((int) mx, 16, 64));
+        mx = max(mx, (uint32_t) __shfl_xor((int) mx, 32, 64));
+        const float qs = ps_scale(mx, qinv);
+        bad |= mx >= 0x7f800000u;
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) {
+            float f[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) f[j] = qf[2 * ks + (j >> 2)][j & 3];
+            ps_split(f, qs, q[ks]);
+        }
+    }
+    f4v o[16];
+#pragma unroll
+    for (int b = 0; b < 16; b++) o[b] = f4v{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.0f;
+    if (ta < tb) {
+        scale_k();
+#pragma unroll
+        for (int i = 0; i < 2; i++) store_k(i);
+        __syncthreads();
+    }
+    for (int ti = ta; ti < tb; ti++) {
+        const int p0 = pfirst + 32 * ti;
+        load_k(p0 + 32);
+        f4v s0[2], s1[2];
+#pragma unroll
+        for (int pb = 0; pb < 2; pb++) s0[pb] = s1[pb] = f4v{0.f, 0.f, 0.f, 0.f};
+        ps_h8 kf[2][2][2];
+        auto read_k = [&](int ks) {
+#pragma unroll
+            for (int pb = 0; pb < 2; pb++)
+#pragma unroll
+                for (int p = 0; p < 2; p++)
+                    kf[ks & 1][pb][p] = *(const ps_h8 *) (ps_lds + p * kPsPlane + (4 * ks + g) * 512 +
+                                                          16 * ((16 * pb + c) ^ ((4 * ks + g) & 15)));
+        };
+        read_k(0);
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) {
+            __builtin_amdgcn_sched_barrier(0);   /* no reads further ahead: no registers */
+            if (ks < 7) read_k(ks + 1);
+#pragma unroll
+            for (int pb = 0; pb < 2; pb++) s1[pb] = ps_mfma(kf[ks & 1][pb][1], q[ks][0], s1[pb]);
+#pragma unroll
+            for (int pb = 0; pb < 2; pb++) s0[pb] = ps_mfma(kf[ks & 1][pb][0], q[ks][0], s0[pb]);
+#pragma unroll
+            for (int pb = 0; pb < 2; pb++) s1[pb] = ps_mfma(kf[ks & 1][pb][0], q[ks][1], s1[pb]);
+            if (ks == 0) scale_v();
+            if (ks >= 3 && ks < 7) store_v(ks - 3);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const f4v ki[2] = {*(const f4v *) (kinv + 4 * g), *(const f4v *) (kinv + 16 + 4 * g)};
+        float e[8];
+        float mc = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 8; i++) e[i] = (s0[i >> 2][i & 3] + s1[i >> 2][i & 3]) * ki[i >> 2][i & 3] * qinv;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int pp = p0 + 16 * (i >> 2) + 4 * g + (i & 3);
+            e[i] = pp >= start_t && pp <= pos_t ? e[i] * scale : -INFINITY;
+            mc = fmaxf(mc, e[i]);
+        }
+        /* the lagging reference maximum of the kernel above */
+        if (__any(mc > m + kPaLag)) {   /* uniform */
+            mc = fmaxf(mc, __shfl_xor(mc, 16, 64));
+            mc = fmaxf(mc, __shfl_xor(mc, 32, 64));
+            const float mn = fmaxf(m, mc);
+            const float a = mn == -INFINITY ? 1.0f : expf(m - mn);
+            l *= a;
+#pragma unroll
+            for (int b = 0; b < 16; b++) o[b] *= a;
+            m = mn;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            e[i] = e[i] == -INFINITY ? 0.0f : expf(e[i] - m);
+            l += e[i];
+        }
+        __syncthreads();   /* V is whole, K read by all */
+        {
+            /* the weights, below e^kPaLag < 2^12, times 2^3 and the quotient of
+             * their V scale to the tile's largest: below 2^15 */
+            const f4v va = *(const f4v *) vinv, vb4 = *(const f4v *) (vinv + 4);
+            const float vmax = fmaxf(fmaxf(fmaxf(va[0], va[1]), fmaxf(va[2], va[3])),
+                                     fmaxf(fmaxf(vb4[0], vb4[1]), fmaxf(vb4[2], vb4[3])));
+            const float vq = __uint_as_float((257u << 23) - __float_as_uint(vmax)), vo = vmax * 0.125f;
+            ps_h8 pw[2];
+            const float w0 = vinv[2 * g] * vq, w1 = vinv[2 * g + 1] * vq;
+#pragma unroll
+            for (int i = 0; i < 8; i++) e[i] *= i < 4 ? w0 : w1;
+            ps_split(e, 1.0f, pw);
+            load_v(p0 + 32);
+            ps_h8 v[2][2][2];
+            auto read_v = [&](int st) {
+#pragma unroll
+                for (int k = 0; k < 2; k++)
+#pragma unroll
+                    for (int p = 0; p < 2; p++)
+                        v[st & 1][k][p] = *(const ps_h8 *) (ps_lds + (2 + p) * kPsPlane + (2 * st + k) * 1024 + 16 * lane);
+            };
+            read_v(0);
+#pragma unroll
+            for (int st = 0; st < 8; st++) {   /* two output blocks a step */
+                __builtin_amdgcn_sched_barrier(0);
+                if (st < 7) read_v(st + 1);
+                f4v r[2];
+#pragma unroll
+                for (int k = 0; k < 2; k++) r[k] = ps_mfma(v[st & 1][k][1], pw[0], f4v{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                for (int k = 0; k < 2; k++) r[k] = ps_mfma(v[st & 1][k][0], pw[1], r[k]);
+#pragma unroll
+                for (int k = 0; k < 2; k++) r[k] = ps_mfma(v[st & 1][k][0], pw[0], r[k]);
+                if (st == 0) scale_k();
+                if (st == 3 || st == 5) store_k((st - 3) / 2);
+#pragma unroll
+                for (int k = 0; k < 2; k++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) o[2 * st + k][i] = __builtin_fmaf(r[k][i], vo, o[2 * st + k][i]);
+            }
+        }
+        __syncthreads();   /* K is whole, V read by all */
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    const bool wbad = __builtin_amdgcn_ballot_w64(bad) != 0;
+    if (lane == 0) flags[wave] = wbad ? 1u : 0u;
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t any = 0;
+        for (int w = 0; w < 8; w++) any |= flags[w];
+        redo[((size_t) z * gridDim.y + t0 / kPsTok) * gridDim.z + kvh] = any;
+    }
+    if (tk >= N) return;
+    const size_t at = ((size_t) z * N + tv) * heads + h;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        f4v * d = (f4v *) (po + at * 256 + 16 * (4 * g + i));
+#pragma unroll
+        for (int k = 0; k < 4; k++) d[k] = f4v{o[4 * k][i], o[4 * k + 1][i], o[4 * k + 2][i], o[4 * k + 3][i]};
+    }
+    if (g == 0) {
+        pml[2 * at] = m;
+        pml[2 * at + 1] = l;
+    }
+}
+
+/* The splits of a token and head in order: outputs and sums brought to the
+ * largest reference, then o / l times the head's sigmoid gate. One wave per
+ * (token, head), four elements per lane. */
+__global__ __launch_bounds__(256) void fw_attn_prompt_merge_kernel(const float * po, const float * pml, int nz, int N,
+                                                                    int heads, const float * gate, int ldg, float * out,
+                                                                    uint16_t * out16) {
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    const int t = blockIdx.x, h = 4 * blockIdx.y + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (h >= heads) return;
+    f4v p[kPsMaxSplit];
+    float ms[kPsMaxSplit], ls[kPsMaxSplit];
+    float mt = -INFINITY;
+#pragma unroll
+    for (int z = 0; z < kPsMaxSplit; z++) {
+        if (z >= nz) continue;   /* uniform */
+        const size_t at = ((size_t) z * N + t) * heads + h;
+        p[z] = *(const f4v *) (po + at * 256 + 4 * lane);
+        ms[z] = pml[2 * at];
+        ls[z] = pml[2 * at + 1];
+        mt = fmaxf(mt, ms[z]);
+    }
+    f4v o = f4v{0.f, 0.f, 0.f, 0.f};
+    float l = 0.0f;
+#pragma unroll
+    for (int z = 0; z < kPsMaxSplit; z++) {
+        if (z >= nz || ms[z] == -INFINITY) continue;
+        const float a = expf(ms[z] - mt);
+        o += p[z] * a;
+        l += ls[z] * a;
+    }
+    const f4v r = o * (1.0f / l) * (1.0f / (1.0f + expf(-gate[(size_t) t * ldg + h])));
+    const size_t ob = ((size_t) t * heads + h) * 256 + 4 * lane;
+    if (out16) {
+        uint2 w;
+        w.x = (uint32_t) fw_bf16(r[0]) | ((uint32_t) fw_bf16(r[1]) << 16);
+        w.y = (uint32_t) fw_bf16(r[2]) | ((uint32_t) fw_bf16(r[3]) << 16);
+        *(uint2 *) (out16 + ob) = w;
+    } else {
+        *(f4v *) (out + ob) = r;
     }
 }
 
@@ -1652,6 +2048,42 @@ int block(Model * m, const uint32_t * tokens, int N, int pos, float * logits, hi
     return kq_gemv_launch(8, m->head_blocks, c.vocab, c.hidden, xin, b16 ? 0 : 1, c.hidden, N, logits, c.vocab, 0, s);
 }
 
+/* Span splits of the split-product prompt attention for a chunk, or 0 where
+ * it does not run: full layers, four query heads per kv head, and a span of
+ * 2048 positions. Below, the partials and two more launches take what the
+ * products save (whole prompt call of the four-layer model, 33 tokens at
+ * 1500: 1155-1184 us without, 1158-1224 with it; 512 at 2000: 1634-1708 and
+ * 1558-1625; 512 at 16384: 2901 and 2050). As many splits as fill the CUs,
+ * leave a split 256 positions and fit the FFN's buffers. */
+int prompt_splits(const Model & m, int N, int pos, int window) {
+    const sparkmv_model_cfg & c = m.c;
+    const int span = pos + N;
+    if (window > 0 || c.heads != 4 * c.kv_heads || span < 2048) return 0;
+    const int wgs = c.kv_heads * ((N + kPsTok - 1) / kPsTok);
+    const size_t one = (size_t) N * (c.heads * 256 + 2 * c.heads) + (size_t) wgs, room = (size_t) (m.vact - m.vmg);
+    int n = (cu_count() + wgs - 1) / wgs;
+    if (n > span / 256) n = span / 256;
+    if (n > kPsMaxSplit) n = kPsMaxSplit;
+    if ((size_t) n * one > room) n = (int) (room / one);
+    return n;
+}
+
+int prompt_split_launch(const float * qkv, int ldq, int kvd, const float * kc, const float * vc, int pos, int N,
+                        int window, int heads, int kv_heads, float scale, int nz, float * po, float * pml,
+                        uint32_t * redo, hipStream_t s) {
+    static std::atomic<int> opted{0};
+    if (!opted.load()) {
+        hipError_t e = hipFuncSetAttribute((const void *) fw_attn_prompt_split_kernel,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, kPsLds);
+        if (e != hipSuccess) return fail_hip("LDS opt-in for the split prompt attention", e);
+        opted.store(1);
+    }
+    hipLaunchKernelGGL(fw_attn_prompt_split_kernel,
+                       dim3((unsigned) nz, (unsigned) ((N + kPsTok - 1) / kPsTok), (unsigned) kv_heads), dim3(512),
+                       kPsLds, s, qkv, ldq, kvd, kc, vc, pos, N, window, heads, scale, po, pml, redo);
+    return check_launch("split prompt attention launch");
+}
+
 /* A prompt chunk (vq-model-gpu.cu:858-943 forward_batch): N tokens at
  * pos .. pos + N - 1 through every layer, the tokens already in m->vtok.
  * With logits, the final norm and the head of the last token
@@ -1693,10 +2125,23 @@ int prompt(Model * m, int N, int pos, float * logits, hipStream_t s) {
         const int window = full ? 0 : c.sliding_window;
         const dim3 ag((unsigned) c.kv_heads, (unsigned) N), ab((unsigned) (64 * (c.heads / c.kv_heads)));
         uint16_t * a16 = b16 ? m->vattn16 : nullptr;
+        const int psplit = hd == 256 ? prompt_splits(*m, N, pos, window) : 0;
+        uint32_t * redo = nullptr;
+        if (psplit > 0) {
+            /* partials in the FFN's buffers, idle here */
+            float * po = m->vmg, * pml = po + (size_t) psplit * N * qd;
+            redo = (uint32_t *) (pml + (size_t) psplit * N * c.heads * 2);
+            if (prompt_split_launch(m->vqkv, ldq, kvd, kc, vc, pos, N, window, c.heads, c.kv_heads, scale, psplit, po,
+                                    pml, redo, s))
+                return -1;
+            hipLaunchKernelGGL(fw_attn_prompt_merge_kernel, dim3((unsigned) N, (unsigned) ((c.heads + 3) / 4)), dim3(256),
+                               0, s, po, pml, psplit, N, c.heads, m->vg, ldq, m->vattn, a16);
+            if (check_launch("prompt attention merge launch")) return -1;
+        }
         if (hd == 256) {
             hipLaunchKernelGGL(fw_attn_prompt_mfma_kernel, dim3((unsigned) c.heads, (unsigned) ((N + kPaTok - 1) / kPaTok)),
                                dim3(256), 0, s, m->vqkv, ldq, kvd, kc, vc, m->vg, ldq, pos, N, window,
-                               c.heads, c.kv_heads, scale, m->vattn, a16);
+                               c.heads, c.kv_heads, scale, m->vattn, a16, (const uint32_t *) redo, psplit);
         }
         else if (hd == 64)
             hipLaunchKernelGGL(fw_attn_prompt_kernel<1>, ag, ab, 0, s, m->vqkv, ldq, kvd, kc, vc, m->vg, ldq, pos,

@@ -528,7 +528,7 @@ static int vq_prefill_impl(const void * const * stages, int nstages, int dim, in
         for (int s0 = 0; s0 < nstages; s0 += 2) {
             const int n = nstages - s0 < 2 ? nstages - s0 : 2;
             if (prefill_mfma_launch(stages + s0, n, L, x, xf32, ldx, 0, ntok, y, ldy, accumulate || s0 > 0,
-                                    (hipStream_t) stream, ws))
+                                    (hipStream_t) stream, ws, kPrefillScratchBytes))
                 return -1;
         }
         return 0;

@@ -1495,6 +1495,10 @@ struct Model {
      * partials for verify blocks of up to 8 tokens */
     void * vmem = nullptr;
     int vcap = 0;
+    /* the prompt matrices' K-split slices, for chunks of up to vcap tokens: a
+     * pool allocation and release per matrix left 20-40 us gaps on the GPU */
+    void * vsplit = nullptr;
+    size_t vsplit_bytes = 0;
     float * vh, * vxn, * vqkv, * vg, * vattn, * vmg, * vmu, * vact, * vpart, * vpml;
     uint16_t * vxn16, * vattn16, * vact16;
     int * vtok;
@@ -1942,6 +1946,17 @@ int alloc_block(Model * m, int cap) {
     const size_t o_part = take((size_t) 8 * c.heads * m->nsplit * c.head_dim * 4);
     const size_t o_pml = take((size_t) 8 * c.heads * m->nsplit * 8);
     const size_t o_tok = take(N * sizeof(int));
+    size_t split = 0;
+    if (cap > kMaxCols) {
+        const int n = cap < kPromptMax ? cap : kPromptMax, ldq = (int) (qd + 2 * kvd);
+        const int shapes[][2] = {{ldq, c.hidden}, {c.heads, c.hidden}, {c.hidden, (int) qd}, {c.intermediate, c.hidden},
+                                 {c.hidden, c.intermediate}};
+        for (const auto & rc : shapes) {
+            const size_t b = prefill_split_bytes(rc[0], rc[1], n);
+            split = b > split ? b : split;
+        }
+    }
+    const size_t o_split = take(split);
     void * mem = nullptr;
     hipError_t e = hipMalloc(&mem, off);
     if (e != hipSuccess) return fail_hip("block buffers", e);
@@ -1949,6 +1964,8 @@ int alloc_block(Model * m, int cap) {
     m->vmem = mem;
     m->vcap = cap;
     uint8_t * b = (uint8_t *) m->vmem;
+    m->vsplit = split ? b + o_split : nullptr;
+    m->vsplit_bytes = split;
     m->vh = (float *) (b + o_h); m->vxn = (float *) (b + o_xn); m->vqkv = (float *) (b + o_qkv);
     m->vg = (float *) (b + o_g); m->vattn = (float *) (b + o_attn); m->vmg = (float *) (b + o_mg);
     m->vmu = (float *) (b + o_mu); m->vact = (float *) (b + o_act); m->vpart = (float *) (b + o_part);
@@ -1969,7 +1986,7 @@ int mat_n(const Model & m, const void * const * st, int rows, int cols, const vo
     const Layout L = make_layout(m.c.dim, m.c.nc, rows, cols, m.c.v3);
     const int xf32 = m.c.x_dtype == SPARKMV_X_F32;
     if (m.c.nstages <= 2 && prefill_mfma_ready(L, m.c.nstages, x, xf32, cols, 0, N))
-        return prefill_mfma_launch(st, m.c.nstages, L, x, xf32, cols, 0, N, y, ldy, acc, s);
+        return prefill_mfma_launch(st, m.c.nstages, L, x, xf32, cols, 0, N, y, ldy, acc, s, m.vsplit, m.vsplit_bytes);
     return prefill_simple_launch(st, m.c.nstages, L, x, xf32, (size_t) cols, 1, N, y, ldy, acc, s);
 }
 

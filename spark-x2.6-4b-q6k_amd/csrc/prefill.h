@@ -19,12 +19,15 @@ int prefill_simple_launch(const void * const * stages, int nst, const Layout & L
  * matrices split K through a stream-ordered workspace and a fixed-order
  * reduction. */
 int prefill_mfma_ready(const Layout & L, int nst, const void * x, int xf32, int ldx, int xt, int ntok);
-/* fixed_ws: NULL takes split slices from the library's pool; otherwise the
- * device address of the no-allocation scratch (prefill_scratch), whose size
- * bounds the split slices. */
+/* fixed_ws: NULL takes split slices from the library's pool; otherwise
+ * fixed_bytes of device memory that bound the split slices: the no-allocation
+ * scratch (prefill_scratch), or a caller's own of prefill_split_bytes. */
 int prefill_mfma_launch(const void * const * stages, int nst, const Layout & L, const void * x, int xf32, int ldx,
                         int xt, int ntok, float * y, int ldy, int accumulate, hipStream_t s,
-                        void * fixed_ws = nullptr);
+                        void * fixed_ws = nullptr, size_t fixed_bytes = 0);
+/* The most bytes of split slices that prefill_mfma_launch takes for rows x
+ * cols and any 1 .. ntok tokens. */
+size_t prefill_split_bytes(int rows, int cols, int ntok);
 
 /* Whether two-stage prefills fold their stages into one f16 weight (the
  * default; off: each stage's exact codewords accumulate apart).

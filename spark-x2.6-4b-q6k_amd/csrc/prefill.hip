@@ -23,6 +23,7 @@
 
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -763,6 +764,15 @@ static int prefill_cw_splits(int rows, int ntok, int nk) {
     return best;
 }
 
+size_t prefill_split_bytes(int rows, int cols, int ntok) {
+    size_t most = 0;
+    for (int n = 1; n <= ntok; n++) {
+        const int S = prefill_cw_splits(rows, n, cols / kPK);
+        if (S > 1) most = std::max(most, (size_t) S * n * rows * sizeof(float));
+    }
+    return most;
+}
+
 static std::atomic<int> g_prefill_fold{1};
 
 int prefill_fold_on() { return g_prefill_fold.load(std::memory_order_relaxed); }
@@ -857,7 +867,7 @@ static int prefill_cw_t(const CwArgs & P, int nsplit, hipStream_t s) {
 
 static int prefill_cw_launch(const void * const * stages, int nst, const Layout & L, const void * x, int xf32,
                              int ldx, int xt, int ntok, float * y, int ldy, int accumulate, hipStream_t s,
-                             void * fixed_ws) {
+                             void * fixed_ws, size_t fixed_bytes) {
     CwArgs P;
     memset(&P, 0, sizeof P);
     P.st[0] = (const uint8_t *) stages[0];
@@ -880,9 +890,9 @@ static int prefill_cw_launch(const void * const * stages, int nst, const Layout 
         if (fixed_ws) {
             /* every slice is written whole by its split before the reduction
              * reads it, so the scratch needs no clearing */
-            if (need > kPrefillScratchBytes) {
+            if (need > fixed_bytes) {
                 set_error("this prefill splits K %d ways and needs %zu bytes of scratch; the no-allocation "
-                          "prefill holds %zu", nsplit, need, (size_t) kPrefillScratchBytes);
+                          "prefill holds %zu", nsplit, need, fixed_bytes);
                 return -1;
             }
             ws = fixed_ws;
@@ -924,14 +934,15 @@ static int prefill_cw_launch(const void * const * stages, int nst, const Layout 
 }
 
 int prefill_mfma_launch(const void * const * stages, int nst, const Layout & L, const void * x, int xf32, int ldx,
-                        int xt, int ntok, float * y, int ldy, int accumulate, hipStream_t s, void * fixed_ws) {
+                        int xt, int ntok, float * y, int ldy, int accumulate, hipStream_t s, void * fixed_ws,
+                        size_t fixed_bytes) {
     if (!prefill_mfma_ready(L, nst, x, xf32, ldx, xt, ntok)) {
         set_error("the MFMA prefill kernel does not take this geometry, stage count or x layout");
         return -1;
     }
     if (ntok <= 0) { set_error("prefill needs at least one token"); return -1; }
     if (prefill_cw_ready(L, nst, x, xf32, ldx, xt, ntok, y, ldy))
-        return prefill_cw_launch(stages, nst, L, x, xf32, ldx, xt, ntok, y, ldy, accumulate, s, fixed_ws);
+        return prefill_cw_launch(stages, nst, L, x, xf32, ldx, xt, ntok, y, ldy, accumulate, s, fixed_ws, fixed_bytes);
     MfmaArgs P;
     memset(&P, 0, sizeof P);
     P.st[0] = (const uint8_t *) stages[0];

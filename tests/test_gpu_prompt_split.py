@@ -75,3 +75,16 @@ def test_infinities_and_nan(sm, ref, dev, which, bad):
     assert np.array_equal(np.isfinite(got), np.isfinite(want))
     ok = np.isfinite(want)
     assert not ok.any() or rel_l2(got[ok], want[ok]) <= 1e-5
+
+
+def test_reservations_grow(sm, ref, dev):
+    """Chunks past a reservation replace the block buffers, the K-split slices
+    with them: 17 tokens reserved and run, then 130, then 20 again."""
+    cfg = dict(BASE, heads=4, kv_heads=1, max_ctx=256)
+    model, oracle = build(sm, ref, dev, "q8_0", sm.X_F32, cfg)
+    model.reserve(17)
+    pos = 0
+    for n in (17, 130, 20):
+        got, want = run(model, oracle, dev, cfg, pos, n)
+        assert rel_l2(got, want) <= 5e-3
+        pos += n

@@ -474,9 +474,8 @@ int sparkmv_model_verify(void * model, const uint32_t * tokens, int ntok, int po
  * skips the head, as forward_batch does between chunks. The host token array
  * is read before the call returns (it waits for the stream's earlier work).
  * Refused past max_ctx or the vocabulary. A chunk longer than the
- * reservation (re)allocates the block buffers after a device
- * synchronization; split-K prefills draw their partial sums from the
- * library's stream-ordered pool (allocated on first use, kept after). */
+ * reservation (re)allocates the block buffers, which also hold split-K
+ * partial sums, after a device synchronization. */
 int sparkmv_model_forward_batch(void * model, const uint32_t * tokens, int ntok, int pos, float * logits,
                                 void * stream);
 /* Allocate the block buffers for verify blocks and prompt chunks of up to

@@ -670,6 +670,13 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : MC == 2 && XF32 ? 512 :
         f4 acc[NA];
 #pragma unroll
         for (int s = 0; s < NA; s++) acc[s] = f4{0.f, 0.f, 0.f, 0.f};
+        /* one-column units of 4 and 9 steps add up in groups of FL, as the
+         * chunks that short matrices ran before did (9 in one sum: 2.2e-7
+         * from the f64 product, 1.4e-7 in groups of 3) */
+        constexpr int FL = MC ? 0 : MSC == 9 ? 3 : MSC == 4 ? 2 : 0;
+        f4 grp[FL ? NST : 1];
+#pragma unroll
+        for (int s = 0; s < (FL ? NST : 1); s++) grp[s] = f4{0.f, 0.f, 0.f, 0.f};
         /* XG: the largest |x| this lane converts in the unit */
         XMax xmx;
         XMax * const xm = XG ? &xmx : nullptr;
@@ -679,6 +686,14 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : MC == 2 && XF32 ? 512 :
                 for (int u = 0; u < D; u++) {
                     mstep<NST, XF32, EXT, XG, 0, LOA>(w[u], cbs, xb + 264 * u, xbl + 264 * u, acc, 1.0f, xm);
                     if (u + kLook < D) ld(w[u + kLook], u + kLook);
+                    if constexpr (FL != 0) {
+                        if ((u + 1) % FL == 0)
+#pragma unroll
+                            for (int s = 0; s < NST; s++) {
+                                grp[s] += acc[s];
+                                acc[s] = u + 1 < D ? f4{0.f, 0.f, 0.f, 0.f} : grp[s];
+                            }
+                    }
                     /* keep step u + kLook's loads here: left to itself the
                      * scheduler sinks them to just before their step, which
                      * then waits a whole memory round trip. (Units of bf16 x from
@@ -1278,11 +1293,15 @@ static int fast_shape_ck(const VqCall & c, int nst, FastShape & sh) {
 }
 
 /* The unit lengths with a straight-line one-column kernel (launch_ms and
- * launch_ms_norm below). */
+ * launch_ms_norm below). 7 and 9 are the parts of rows of 1792, 3584, 7168 and
+ * of 1152, 2304, 4608, 9216 columns (one column of 3584 x 3584 12.0 -> 8.7 us,
+ * of 2304 x 9216 27.3 -> 9.3 against the ring form). 13-bit units stop at 8
+ * steps: longer ones would spill. */
 static int straight_ms(int MS, int ext, int norm) {
     switch (MS) {
         case 1: case 2: case 4: case 5: case 8: return 1;
-        case 3: case 6: return !norm;
+        case 3: case 6: case 7: return !norm;
+        case 9: return !norm && !ext;
         case 10: return !ext;
         default: return 0;
     }
@@ -1428,7 +1447,7 @@ static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
     return 0;
 }
 
-/* Units of 1-6, 8 or 10 macro steps (the trunk's shapes give 2, 5 and 10;
+/* Units of 1 to 10 macro steps (the trunk's shapes give 2, 5 and 10;
  * several columns 2, 4, 5, 8 or 10) run the straight-line kernels; any other
  * length the ring kernel. Thirteen-bit indices hold plane bytes too, so their
  * straight-line units stop at 8 steps (10 would spill). */
@@ -1516,6 +1535,8 @@ static int launch_ms(const FastArgs & A, int MS, int mc, int grid, int threads, 
             case 4: return launch_fast_t<NST, 0, EXT, 4>(A, grid, threads, lds, s);
             case 5: return launch_fast_t<NST, 0, EXT, 5>(A, grid, threads, lds, s);
             case 6: return launch_fast_t<NST, 0, EXT, 6>(A, grid, threads, lds, s);
+            case 7: return launch_fast_t<NST, 0, EXT, 7>(A, grid, threads, lds, s);
+            case 9: if (!EXT) return launch_fast_t<NST, 0, EXT, EXT ? 0 : 9>(A, grid, threads, lds, s); break;
             case 8: return launch_fast_t<NST, 0, EXT, 8>(A, grid, threads, lds, s);
             case 10: if (!EXT) return launch_fast_t<NST, 0, EXT, EXT ? 0 : 10>(A, grid, threads, lds, s); break;
             default: break;
@@ -1530,6 +1551,8 @@ static int launch_ms(const FastArgs & A, int MS, int mc, int grid, int threads, 
             case 4: return launch_fast_t<NST, 1, EXT, 4>(A, grid, threads, lds, s);
             case 5: return launch_fast_t<NST, 1, EXT, 5>(A, grid, threads, lds, s);
             case 6: return launch_fast_t<NST, 1, EXT, 6>(A, grid, threads, lds, s);
+            case 7: return launch_fast_t<NST, 1, EXT, 7>(A, grid, threads, lds, s);
+            case 9: if (!EXT) return launch_fast_t<NST, 1, EXT, EXT ? 0 : 9>(A, grid, threads, lds, s); break;
             case 8: return launch_fast_t<NST, 1, EXT, 8>(A, grid, threads, lds, s);
             case 10: if (!EXT) return launch_fast_t<NST, 1, EXT, EXT ? 0 : 10>(A, grid, threads, lds, s); break;
             default: break;

@@ -84,7 +84,7 @@ def test_f32_columns_spike_and_non_finite(sm, ref, dev, cols):
 @pytest.mark.parametrize("f32", [False, True], ids=["bf16x", "f32x"])
 @pytest.mark.parametrize("rows,cols,nc", [(1024, 2560, 4096), (8, 256, 4096), (520, 10240, 4096), (16, 10240, 4096),
                                           (1024, 4096, 4096), (600, 1152, 4096), (300, 8192, 8192), (40, 2560, 4094),
-                                          (64, 2560, 1 << 12)])
+                                          (64, 2560, 1 << 12), (2304, 2304, 4096), (600, 1792, 4096), (70, 1152, 4096), (96, 1152, 8192)])
 def test_one_column_of_a_short_matrix(sm, ref, dev, rows, cols, nc, f32):
     import torch
     data = sm.synth_container(rows + cols, rows, cols, 4, nc, 2, 1)

@@ -1068,16 +1068,24 @@ __global__ __launch_bounds__(256) void fw_attn_prompt_mfma_kernel(const float * 
 /* Prompt attention over long spans, for 256-element heads in groups of four
  * query heads per kv head: the products on the f16 matrix cores, f32 in
  * value. Every f32 operand is brought to the top of f16's range by a power of
- * two (exact: per token for q, per position for k, per four positions for v,
- * whose weights take the quotient to the tile's largest) and split into two
- * f16 halves, hi + lo = x to 2^-23 of x; hi hi, hi lo and lo hi are taken (lo
- * lo is below 2^-24). Three f16 products run in 3/16 of the f32 products'
- * matrix-core time. Sums stay f32: hi hi and the small products of the scores
- * have an accumulator each, and the outputs of 32 positions are summed apart,
- * small products first, then added to the running output: it rounds once per
- * 32 positions (the f32 kernel above, every 4). Distance of f32 logits from
- * the 64-bit ones, both within 0.5 % of each other: 1.34e-6 (12 tokens at
- * 3000), 2.03e-6 (16 at 16000).
+ * two (exact) and split into two f16 halves; hi hi, hi lo and lo hi are taken
+ * (lo lo is below 2^-24). q has a scale per token, k and v one per position,
+ * and the weights, times their rows' v scales, one per token and tile, which
+ * the token's output column carries back. No scale is shared between
+ * positions, so what a token does not see (or weighs little) takes no bits
+ * from what it sees. hi + lo is x to 2^-23 of x, or to 2^-39 of the largest
+ * operand under the same scale where x is below 2^-16 of it: of the largest
+ * element of the same row, or, for a weight, of the token's largest in the
+ * tile. (The out matvec that reads the result splits all of a token's heads
+ * under one scale in the same way.) Three f16 products run in 3/16 of the f32
+ * products' matrix-core time. Sums stay f32: hi hi and the small products of
+ * the scores have an accumulator each, and the outputs of 32 positions are
+ * summed apart, small products first, then added to the running output: it
+ * rounds once per 32 positions (the f32 kernel above, every 4). Distance of
+ * 16 tokens' rows from 64 bits, mean, f32 kernel and here: 1.0e-6 and 1.2e-6
+ * at 2070 with sharp scores (deviation 6), 8.0e-7 and 6.9e-7 there with
+ * deviation 2, 1.5e-6 and 1.1e-6 at 16000; values of one sign 4.9e-7 and
+ * 2.0e-7 there.
  *
  * One workgroup per (kv head, 32 tokens, span split): of its eight waves,
  * wave w is query head w % 4 of the group and tokens 16 (w / 4) .. against all
@@ -1093,7 +1101,9 @@ __global__ __launch_bounds__(256) void fw_attn_prompt_mfma_kernel(const float * 
  * of the time). Nothing may spill here: a wave's loads return in order, so a
  * reload in the loop waits for the K and V requests before it (59 spilled
  * registers: 1400 us). Three bf16 planes and six products need no scales but
- * spilled, at 1390 us.
+ * spilled, at 1390 us. Scales per v row and per token cost 5 us of 592 against
+ * one v scale per tile, which lost the weights of rows beside a much larger
+ * or an all-zero one.
  *
  * Layouts (16x16x32: lane l = 16 g + c holds A[c][8 g + j], B[8 g + j][c],
  * D[4 g + i][c]): scores are positions x tokens, so a lane's 8 weights are of
@@ -1105,7 +1115,7 @@ __global__ __launch_bounds__(256) void fw_attn_prompt_mfma_kernel(const float * 
  * block][kv head], and the f32 kernel above then does those blocks again. */
 constexpr int kPsTok = 32;                          /* tokens per workgroup, positions per tile */
 constexpr int kPsPlane = 16384;                     /* LDS bytes of one half of a tile */
-constexpr int kPsLds = 4 * kPsPlane + 256;          /* K and V halves, scales, the waves' flags */
+constexpr int kPsLds = 4 * kPsPlane + 320;          /* K and V halves, scales, the waves' flags */
 constexpr int kPsMaxSplit = 8;
 
 typedef uint32_t ps_u4 __attribute__((ext_vector_type(4)));
@@ -1129,10 +1139,21 @@ static __device__ __forceinline__ uint32_t ps_max16(uint32_t m) {
     return max(m, (uint32_t) __builtin_amdgcn_update_dpp(0, (int) m, 0x140, 0xf, 0xf, false)); /* in 16 */
 }
 
+/* The largest of m over the lanes l, l ^ 16, l ^ 32 and l ^ 48, in each of
+ * them: register swaps (odd rows of 16 lanes with even ones, then halves of
+ * the wave), no LDS round trip ahead of the output products */
+static __device__ __forceinline__ uint32_t ps_max_rows(uint32_t m) {
+    const auto a = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+    m = max(a[0], a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+    return max(b[0], b[1]);
+}
+
 /* The power of two that brings the largest magnitude (f32 bits) to [2^14,
- * 2^15), and its inverse */
+ * 2^15) (as far as 2^126 takes it), and its inverse; zero gives the smallest
+ * inverse, so that nothing is scaled down for it */
 static __device__ __forceinline__ float ps_scale(uint32_t mag, float & inv) {
-    const uint32_t f = mag == 0u ? 127u : min(268u - min(mag >> 23, 254u), 253u);
+    const uint32_t f = min(268u - min(mag >> 23, 254u), 253u);
     inv = __uint_as_float((254u - f) << 23);
     return __uint_as_float(f << 23);
 }
@@ -1145,23 +1166,21 @@ static __device__ __forceinline__ ps_f4 ps_mfma(ps_h8 a, ps_h8 b, ps_f4 c) {
 
 __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float * qkv, int ldq, int kvd,
                                                                     const float * kc, const float * vc, int pos0, int N,
-                                                                    int window, int heads, float scale, float * po,
-                                                                    float * pml, uint32_t * redo) {
+                                                                    int heads, float scale, float * po, float * pml,
+                                                                    uint32_t * redo) {
     typedef ps_f4 f4v;
     typedef _Float16 h4v __attribute__((ext_vector_type(4)));
     extern __shared__ __attribute__((aligned(16))) uint8_t ps_lds[];
     float * kinv = (float *) (ps_lds + 4 * kPsPlane);          /* K's inverse scale per position */
-    float * vinv = kinv + 32;                                  /* V's per four positions 16 pb + 4 g .., at [2 g + pb] */
-    uint32_t * flags = (uint32_t *) (vinv + 8);                /* per wave, at the end */
+    float * vinv = kinv + 32;                                  /* V's */
+    uint32_t * flags = (uint32_t *) (vinv + 32);               /* per wave, at the end */
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, c = lane & 15;
     /* the blocks with the longest causal range first */
     const int kvh = blockIdx.z, t0 = ((int) gridDim.y - 1 - (int) blockIdx.y) * kPsTok, h = 4 * kvh + (wave & 3);
     const int tk = t0 + 16 * (wave >> 2) + c;
     const int tv = min(tk, N - 1), pos_t = pos0 + tv;
-    const int start_t = window > 0 && pos_t + 1 > window ? pos_t + 1 - window : 0;
-    const int pfirst = window > 0 && pos0 + t0 + 1 > window ? pos0 + t0 + 1 - window : 0;
     const int plast = pos0 + min(t0 + kPsTok - 1, N - 1);
-    const int nt = (plast - pfirst) / 32 + 1, nz = gridDim.x, z = blockIdx.x;
+    const int nt = plast / 32 + 1, nz = gridDim.x, z = blockIdx.x;
     const int ta = (int) ((long) nt * z / nz), tb = (int) ((long) nt * (z + 1) / nz);
     const float * kb = kc + (size_t) kvh * 256, * vb = vc + (size_t) kvh * 256;
     const float * qrow = qkv + (size_t) tv * ldq + (size_t) h * 256;
@@ -1216,27 +1235,32 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
         for (int j = 0; j < 4; j++)
             vr[j] = *(const f4v *) (vb + (size_t) min(p0 + 16 * vp + 4 * vg + j, plast) * kvd + 4 * lane);
     };
-    float vsc = 1.0f;
+    float vsc[4];
     auto scale_v = [&]() {
-        uint32_t m = 0;
+        uint32_t all = 0;
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < 4; j++) {
+            uint32_t m = 0;
 #pragma unroll
             for (int e = 0; e < 4; e++) m = max(m, __float_as_uint(vr[j][e]) & 0x7fffffffu);
-        m = ps_max16(m);
-        m = max(m, (uint32_t) __shfl_xor((int) m, 16, 64));
-        m = max(m, (uint32_t) __shfl_xor((int) m, 32, 64));
-        float inv;
-        vsc = ps_scale(m, inv);
-        if (lane == 0) vinv[wave] = inv;
-        bad |= m >= 0x7f800000u;
+            m = ps_max16(m);
+            /* the row's largest in a scalar register, its scale with it */
+            uint32_t w = 0;
+#pragma unroll
+            for (int r = 0; r < 4; r++) w = max(w, (uint32_t) __builtin_amdgcn_readlane((int) m, 16 * r));
+            all = max(all, w);
+            float inv;
+            vsc[j] = ps_scale(w, inv);
+            if (lane == 0) vinv[16 * vp + 4 * vg + j] = inv;
+        }
+        bad |= all >= 0x7f800000u;
     };
     /* element 4 lane + e is row lane / 4 of block 4 (lane % 4) + e */
     auto store_v = [&](int e) {
         h4v hi, lo;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const float x = vr[j][e] * vsc;
+            const float x = vr[j][e] * vsc[j];
             hi[j] = (_Float16) x;
             lo[j] = (_Float16) (x - (float) hi[j]);
         }
@@ -1246,8 +1270,8 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
     };
 
     if (ta < tb) {
-        load_k(pfirst + 32 * ta);
-        load_v(pfirst + 32 * ta);
+        load_k(32 * ta);
+        load_v(32 * ta);
     }
     /* the token's query: halves of the row's 8 steps, the row's scale over the
      * four lanes that hold it */
@@ -1285,7 +1309,7 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
         __syncthreads();
     }
     for (int ti = ta; ti < tb; ti++) {
-        const int p0 = pfirst + 32 * ti;
+        const int p0 = 32 * ti;
         load_k(p0 + 32);
         f4v s0[2], s1[2];
 #pragma unroll
@@ -1322,7 +1346,7 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int pp = p0 + 16 * (i >> 2) + 4 * g + (i & 3);
-            e[i] = pp >= start_t && pp <= pos_t ? e[i] * scale : -INFINITY;
+            e[i] = pp <= pos_t ? e[i] * scale : -INFINITY;
             mc = fmaxf(mc, e[i]);
         }
         /* the lagging reference maximum of the kernel above */
@@ -1343,17 +1367,22 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
         }
         __syncthreads();   /* V is whole, K read by all */
         {
-            /* the weights, below e^kPaLag < 2^12, times 2^3 and the quotient of
-             * their V scale to the tile's largest: below 2^15 */
-            const f4v va = *(const f4v *) vinv, vb4 = *(const f4v *) (vinv + 4);
-            const float vmax = fmaxf(fmaxf(fmaxf(va[0], va[1]), fmaxf(va[2], va[3])),
-                                     fmaxf(fmaxf(vb4[0], vb4[1]), fmaxf(vb4[2], vb4[3])));
-            const float vq = __uint_as_float((257u << 23) - __float_as_uint(vmax)), vo = vmax * 0.125f;
-            ps_h8 pw[2];
-            const float w0 = vinv[2 * g] * vq, w1 = vinv[2 * g + 1] * vq;
+            /* the token's weights in units of its V rows' scales, brought to the
+             * top of f16's range by a power of two of the token's own: only
+             * what it sees has a weight. e^kPaLag < 2^12 and inverse scales of
+             * at most 2^113 stay finite */
+            const f4v va[2] = {*(const f4v *) (vinv + 4 * g), *(const f4v *) (vinv + 16 + 4 * g)};
+            uint32_t wm = 0;
 #pragma unroll
-            for (int i = 0; i < 8; i++) e[i] *= i < 4 ? w0 : w1;
-            ps_split(e, 1.0f, pw);
+            for (int i = 0; i < 8; i++) {
+                e[i] *= va[i >> 2][i & 3];
+                wm = max(wm, __float_as_uint(e[i]));
+            }
+            wm = ps_max_rows(wm);
+            float vo;
+            const float ws = ps_scale(wm, vo);
+            ps_h8 pw[2];
+            ps_split(e, ws, pw);
             load_v(p0 + 32);
             ps_h8 v[2][2][2];
             auto read_v = [&](int st) {
@@ -2086,8 +2115,8 @@ int prompt_splits(const Model & m, int N, int pos, int window) {
 }
 
 int prompt_split_launch(const float * qkv, int ldq, int kvd, const float * kc, const float * vc, int pos, int N,
-                        int window, int heads, int kv_heads, float scale, int nz, float * po, float * pml,
-                        uint32_t * redo, hipStream_t s) {
+                        int heads, int kv_heads, float scale, int nz, float * po, float * pml, uint32_t * redo,
+                        hipStream_t s) {
     static std::atomic<int> opted{0};
     if (!opted.load()) {
         hipError_t e = hipFuncSetAttribute((const void *) fw_attn_prompt_split_kernel,
@@ -2097,7 +2126,7 @@ int prompt_split_launch(const float * qkv, int ldq, int kvd, const float * kc, c
     }
     hipLaunchKernelGGL(fw_attn_prompt_split_kernel,
                        dim3((unsigned) nz, (unsigned) ((N + kPsTok - 1) / kPsTok), (unsigned) kv_heads), dim3(512),
-                       kPsLds, s, qkv, ldq, kvd, kc, vc, pos, N, window, heads, scale, po, pml, redo);
+                       kPsLds, s, qkv, ldq, kvd, kc, vc, pos, N, heads, scale, po, pml, redo);
     return check_launch("split prompt attention launch");
 }
 
@@ -2148,8 +2177,8 @@ int prompt(Model * m, int N, int pos, float * logits, hipStream_t s) {
             /* partials in the FFN's buffers, idle here */
             float * po = m->vmg, * pml = po + (size_t) psplit * N * qd;
             redo = (uint32_t *) (pml + (size_t) psplit * N * c.heads * 2);
-            if (prompt_split_launch(m->vqkv, ldq, kvd, kc, vc, pos, N, window, c.heads, c.kv_heads, scale, psplit, po,
-                                    pml, redo, s))
+            if (prompt_split_launch(m->vqkv, ldq, kvd, kc, vc, pos, N, c.heads, c.kv_heads, scale, psplit, po, pml,
+                                    redo, s))
                 return -1;
             hipLaunchKernelGGL(fw_attn_prompt_merge_kernel, dim3((unsigned) N, (unsigned) ((c.heads + 3) / 4)), dim3(256),
                                0, s, po, pml, psplit, N, c.heads, m->vg, ldq, m->vattn, a16);

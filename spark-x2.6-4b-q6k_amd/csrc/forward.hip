@@ -1150,13 +1150,16 @@ static __device__ __forceinline__ uint32_t ps_max_rows(uint32_t m) {
 }
 
 /* The power of two that brings the largest magnitude (f32 bits) to [2^14,
- * 2^15) (as far as 2^126 takes it), and its inverse; zero gives the smallest
- * inverse, so that nothing is scaled down for it */
-static __device__ __forceinline__ float ps_scale(uint32_t mag, float & inv) {
+ * 2^15) (as far as 2^126 takes it), and its inverse's exponent, -126 .. 113;
+ * zero gives the smallest, so that nothing is scaled down for it */
+static __device__ __forceinline__ float ps_scale(uint32_t mag, int & ex) {
     const uint32_t f = min(268u - min(mag >> 23, 254u), 253u);
-    inv = __uint_as_float((254u - f) << 23);
+    ex = 127 - (int) f;
     return __uint_as_float(f << 23);
 }
+
+/* 2^ex, ex in -126 .. 127 */
+static __device__ __forceinline__ float ps_pow2(int ex) { return __uint_as_float((uint32_t) (ex + 127) << 23); }
 
 typedef float ps_f4 __attribute__((ext_vector_type(4)));
 
@@ -1169,12 +1172,15 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
                                                                     int heads, float scale, float * po, float * pml,
                                                                     uint32_t * redo) {
     typedef ps_f4 f4v;
+    typedef int i4v __attribute__((ext_vector_type(4)));
     typedef _Float16 h4v __attribute__((ext_vector_type(4)));
     extern __shared__ __attribute__((aligned(16))) uint8_t ps_lds[];
-    float * kinv = (float *) (ps_lds + 4 * kPsPlane);          /* K's inverse scale per position */
-    float * vinv = kinv + 32;                                  /* V's */
+    int * kexp = (int *) (ps_lds + 4 * kPsPlane);              /* exponent of K's inverse scale per position */
+    float * vinv = (float *) (kexp + 32);                      /* V's inverse scale */
     uint32_t * flags = (uint32_t *) (vinv + 32);               /* per wave, at the end */
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, c = lane & 15;
+    /* the wave as a scalar: what depends on it alone takes no vector register */
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, g = lane >> 4, c = lane & 15;
     /* the blocks with the longest causal range first */
     const int kvh = blockIdx.z, t0 = ((int) gridDim.y - 1 - (int) blockIdx.y) * kPsTok, h = 4 * kvh + (wave & 3);
     const int tk = t0 + 16 * (wave >> 2) + c;
@@ -1210,9 +1216,9 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
             m = ps_max16(m);
             m = max(m, (uint32_t) __shfl_xor((int) m, 16, 64));
             all = max(all, m);
-            float inv;
-            ksc[i] = ps_scale(m, inv);
-            if (kg == 0) kinv[16 * i + kp] = inv;
+            int ex;
+            ksc[i] = ps_scale(m, ex);
+            if (kg == 0) kexp[16 * i + kp] = ex;
         }
         bad |= all >= 0x7f800000u;
     };
@@ -1249,9 +1255,9 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
 #pragma unroll
             for (int r = 0; r < 4; r++) w = max(w, (uint32_t) __builtin_amdgcn_readlane((int) m, 16 * r));
             all = max(all, w);
-            float inv;
-            vsc[j] = ps_scale(w, inv);
-            if (lane == 0) vinv[16 * vp + 4 * vg + j] = inv;
+            int ex;
+            vsc[j] = ps_scale(w, ex);
+            if (lane == 0) vinv[16 * vp + 4 * vg + j] = ps_pow2(ex);
         }
         bad |= all >= 0x7f800000u;
     };
@@ -1276,7 +1282,7 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
     /* the token's query: halves of the row's 8 steps, the row's scale over the
      * four lanes that hold it */
     ps_h8 q[8][2];
-    float qinv;
+    int qexp;
     {
         f4v qf[16];
         uint32_t mx = 0;
@@ -1288,7 +1294,7 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
         }
         mx = max(mx, (uint32_t) __shfl_xor((int) mx, 16, 64));
         mx = max(mx, (uint32_t) __shfl_xor((int) mx, 32, 64));
-        const float qs = ps_scale(mx, qinv);
+        const float qs = ps_scale(mx, qexp);
         bad |= mx >= 0x7f800000u;
 #pragma unroll
         for (int ks = 0; ks < 8; ks++) {
@@ -1338,11 +1344,13 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
             if (ks >= 3 && ks < 7) store_v(ks - 3);
         }
         __builtin_amdgcn_sched_barrier(0);
-        const f4v ki[2] = {*(const f4v *) (kinv + 4 * g), *(const f4v *) (kinv + 16 + 4 * g)};
+        const i4v ki[2] = {*(const i4v *) (kexp + 4 * g), *(const i4v *) (kexp + 16 + 4 * g)};
         float e[8];
         float mc = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < 8; i++) e[i] = (s0[i >> 2][i & 3] + s1[i >> 2][i & 3]) * ki[i >> 2][i & 3] * qinv;
+        for (int i = 0; i < 8; i++)
+            /* both scales in one step: a large key's alone may pass f32's range */
+            e[i] = __builtin_ldexpf(s0[i >> 2][i & 3] + s1[i >> 2][i & 3], ki[i >> 2][i & 3] + qexp);
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int pp = p0 + 16 * (i >> 2) + 4 * g + (i & 3);
@@ -1379,8 +1387,8 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
                 wm = max(wm, __float_as_uint(e[i]));
             }
             wm = ps_max_rows(wm);
-            float vo;
-            const float ws = ps_scale(wm, vo);
+            int wexp;
+            const float ws = ps_scale(wm, wexp), vo = ps_pow2(wexp);
             ps_h8 pw[2];
             ps_split(e, ws, pw);
             load_v(p0 + 32);

@@ -214,3 +214,12 @@ def test_small_rows_with_the_weight(sm, ref, dev, vexp):
     V[64:68] = np.ldexp(V[64:68], vexp)
     err = every_token(model, cfg, want, dev, toks, pos, K, V)
     assert max(err) <= 1e-5, err
+
+
+@pytest.mark.parametrize("kexp", [20, 100, 109, 114])
+def test_large_keys_and_small_queries(sm, ref, dev, kexp):
+    """Scores of order 1 to 8 whose keys alone, times the query's scaled halves, pass f32's range."""
+    model, cfg, want = one_layer(sm, ref, dev, gain=2.0 ** (3 - kexp))
+    rng, pos = np.random.default_rng(5), 2070
+    err = every_token(model, cfg, want, dev, list(range(9)), pos, rows(rng, pos, kexp), rows(rng, pos, 0, 1.0))
+    assert max(err) <= 1e-5, err

@@ -1078,14 +1078,15 @@ __global__ __launch_bounds__(256) void fw_attn_prompt_mfma_kernel(const float * 
  * element of the same row, or, for a weight, of the token's largest in the
  * tile. (The out matvec that reads the result splits all of a token's heads
  * under one scale in the same way.) Three f16 products run in 3/16 of the f32
- * products' matrix-core time. Sums stay f32: hi hi and the small products of
- * the scores have an accumulator each, and the outputs of 32 positions are
- * summed apart, small products first, then added to the running output: it
- * rounds once per 32 positions (the f32 kernel above, every 4). Distance of
- * 16 tokens' rows from 64 bits, mean, f32 kernel and here: 1.0e-6 and 1.2e-6
- * at 2070 with sharp scores (deviation 6), 8.0e-7 and 6.9e-7 there with
- * deviation 2, 1.5e-6 and 1.1e-6 at 16000; values of one sign 4.9e-7 and
- * 2.0e-7 there.
+ * products' matrix-core time. Sums stay f32: the scores' hi hi products have
+ * two accumulators, their small products one (one and one rounded often enough
+ * at the size of the score to show in sharp weights), and the outputs of 32
+ * positions are summed apart, small products first, then added to the running
+ * output: it rounds once per 32 positions (the f32 kernel above, every 4).
+ * Distance of a token's row from 64 bits, mean of 160, f32 kernel and here (one
+ * hi hi accumulator): scores of deviation 3 at position 2070 8.5e-7 and 6.3e-7
+ * (8.0e-7), of 12 there 1.10e-6 and 1.02e-6 (1.26e-6), at 3000 1.12e-6 and
+ * 9.3e-7 (1.20e-6).
  *
  * One workgroup per (kv head, 32 tokens, span split): of its eight waves,
  * wave w is query head w % 4 of the group and tokens 16 (w / 4) .. against all
@@ -1095,15 +1096,16 @@ __global__ __launch_bounds__(256) void fw_attn_prompt_mfma_kernel(const float * 
  * registers each) stay in registers; K is converted while the outputs' MFMAs
  * run, V while the scores' do, each requested a phase earlier.
  *
- * 512 tokens at 16384, 16 heads: 592 us, 1378 in the f32 kernel (101 TFLOP/s
- * of f32 products; 236 here). What bounds it is the conversions' and
+ * 512 tokens at 16384, 16 heads: 610 us, 1378 in the f32 kernel (101 TFLOP/s
+ * of f32 products; 229 here). What bounds it is the conversions' and
  * softmax's VALU work and the two barriers per tile (MFMAs are busy a quarter
  * of the time). Nothing may spill here: a wave's loads return in order, so a
  * reload in the loop waits for the K and V requests before it (59 spilled
  * registers: 1400 us). Three bf16 planes and six products need no scales but
- * spilled, at 1390 us. Scales per v row and per token cost 5 us of 592 against
- * one v scale per tile, which lost the weights of rows beside a much larger
- * or an all-zero one.
+ * spilled, at 1390 us. Scales per v row and per token, exponents for keys and
+ * queries and the second accumulator cost 18 us of 592 against one v scale per
+ * tile, which lost the weights of rows beside a much larger or an all-zero one.
+ * Taking lo lo too costs 28 us more and gains 2 % of the distance.
  *
  * Layouts (16x16x32: lane l = 16 g + c holds A[c][8 g + j], B[8 g + j][c],
  * D[4 g + i][c]): scores are positions x tokens, so a lane's 8 weights are of
@@ -1317,9 +1319,9 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
     for (int ti = ta; ti < tb; ti++) {
         const int p0 = 32 * ti;
         load_k(p0 + 32);
-        f4v s0[2], s1[2];
+        f4v s0[2][2], s1[2];
 #pragma unroll
-        for (int pb = 0; pb < 2; pb++) s0[pb] = s1[pb] = f4v{0.f, 0.f, 0.f, 0.f};
+        for (int pb = 0; pb < 2; pb++) s0[pb][0] = s0[pb][1] = s1[pb] = f4v{0.f, 0.f, 0.f, 0.f};
         ps_h8 kf[2][2][2];
         auto read_k = [&](int ks) {
 #pragma unroll
@@ -1337,7 +1339,7 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
 #pragma unroll
             for (int pb = 0; pb < 2; pb++) s1[pb] = ps_mfma(kf[ks & 1][pb][1], q[ks][0], s1[pb]);
 #pragma unroll
-            for (int pb = 0; pb < 2; pb++) s0[pb] = ps_mfma(kf[ks & 1][pb][0], q[ks][0], s0[pb]);
+            for (int pb = 0; pb < 2; pb++) s0[pb][ks & 1] = ps_mfma(kf[ks & 1][pb][0], q[ks][0], s0[pb][ks & 1]);
 #pragma unroll
             for (int pb = 0; pb < 2; pb++) s1[pb] = ps_mfma(kf[ks & 1][pb][0], q[ks][1], s1[pb]);
             if (ks == 0) scale_v();
@@ -1350,7 +1352,7 @@ __global__ __launch_bounds__(512) void fw_attn_prompt_split_kernel(const float *
 #pragma unroll
         for (int i = 0; i < 8; i++)
             /* both scales in one step: a large key's alone may pass f32's range */
-            e[i] = __builtin_ldexpf(s0[i >> 2][i & 3] + s1[i >> 2][i & 3], ki[i >> 2][i & 3] + qexp);
+            e[i] = __builtin_ldexpf((s0[i >> 2][0][i & 3] + s0[i >> 2][1][i & 3]) + s1[i >> 2][i & 3], ki[i >> 2][i & 3] + qexp);
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int pp = p0 + 16 * (i >> 2) + 4 * g + (i & 3);

@@ -95,7 +95,7 @@ def test_reservations_grow(sm, ref, dev):
         pos += n
 
 
-def one_layer(sm, ref, dev, heads=4, kvh=1, eps=1e-20, gain=1.0, zero=(), loud=()):
+def one_layer(sm, ref, dev, heads=4, kvh=1, eps=1e-20, gain=1.0, zero=(), loud=(), inter=BASE["intermediate"]):
     """A full layer whose attention output reaches the next layer's input
     unmixed: its MLP adds nothing (a zero norm) and the embedding is faint,
     2^-18, or zero for tokens of `zero` (no query, key, value or residual) and
@@ -104,8 +104,8 @@ def one_layer(sm, ref, dev, heads=4, kvh=1, eps=1e-20, gain=1.0, zero=(), loud=(
     embedding, of that of gain * 2^-18 / sqrt(eps). Returns the model, which
     captures that input at slot 1, and the same in f64."""
     import torch
-    c = dict(BASE, heads=heads, kv_heads=kvh, eps=eps, layers=2)
-    hid, hd, inter = c["hidden"], c["head_dim"], c["intermediate"]
+    c = dict(BASE, heads=heads, kv_heads=kvh, eps=eps, layers=2, intermediate=inter)
+    hid, hd = c["hidden"], c["head_dim"]
     qd, kvd = heads * hd, kvh * hd
     shapes = dict(qkv=(qd + 2 * kvd, hid), attn_gate=(heads, hid), out=(hid, qd), gate=(inter, hid), up=(inter, hid),
                   down=(hid, inter))
@@ -223,3 +223,20 @@ def test_large_keys_and_small_queries(sm, ref, dev, kexp):
     rng, pos = np.random.default_rng(5), 2070
     err = every_token(model, cfg, want, dev, list(range(9)), pos, rows(rng, pos, kexp), rows(rng, pos, 0, 1.0))
     assert max(err) <= 1e-5, err
+
+
+@pytest.mark.parametrize("width,mean", [(0.5, 0.0), (6, 0.0), (12, 0.0), (12, 1.0)])
+def test_no_further_from_64_bits_than_the_f32_kernel(sm, ref, dev, width, mean):
+    """Chunks of 16 tokens through this kernel and, under an FFN too narrow
+    for its partials, through the f32 one, over scores of deviation `width`
+    (sharp ones show their last bits in the weights)."""
+    pos, err = 2070, []
+    for inter in (BASE["intermediate"], 512):
+        model, cfg, want = one_layer(sm, ref, dev, inter=inter)
+        total = 0.0
+        for seed in range(6):
+            rng = np.random.default_rng(seed)
+            K, V = rows(rng, pos, 0) * np.float32(width / 0.47), rows(rng, pos, 0, mean)
+            total += sum(every_token(model, cfg, want, dev, rng.integers(0, cfg["vocab"], 16).tolist(), pos, K, V))
+        err.append(total)
+    assert err[0] <= err[1], err

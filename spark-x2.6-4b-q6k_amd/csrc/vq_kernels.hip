@@ -1399,8 +1399,11 @@ static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
          * the codebooks in one pass of five chunks per thread and stage (and
          * x in two), which the straight-line kernels ask for and the ring
          * form is slow without: waves past the tiles stage and then end. One
-         * f32 column of 1024 x 2560 22.0 -> 8.9 us. */
-        sh.W = std::max(sh.W, std::max(std::min(10, (n16 + 319) / 320), std::min(10, (c.cols + 1023) / 1024)));
+         * f32 column of 1024 x 2560 22.0 -> 8.9 us. As many as LDS holds:
+         * x that fits without them stays in one K range (two 13-bit
+         * codebooks beside one f32 column of 5376 to 7552). */
+        const int wmax = std::max(std::min(10, (n16 + 319) / 320), std::min(10, (c.cols + 1023) / 1024));
+        while (sh.W < wmax && fast_lds(c, nst, S, sh.W + 1) <= (size_t) kLdsMax) sh.W++;
     }
     sh.nwg = 0;
     for (int m = 0; m < c.nmat; m++) sh.nwg += (int) (((c.mats[m].rows * (long) S + 15) / 16 + T - 1) / T);

@@ -95,3 +95,33 @@ def test_one_column_of_a_short_matrix(sm, ref, dev, rows, cols, nc, f32):
     sm.DeviceContainer(data).gemv(xt, y)
     torch.cuda.synchronize()
     assert rel_l2(y[0].cpu().numpy(), W @ xt[0].double().cpu().numpy()) <= TIGHT
+
+
+def launches(stream, call):
+    """Kernels that call() puts on the stream, from a capture of it."""
+    import ctypes
+    hip, graph, n = ctypes.CDLL("libamdhip64.so"), ctypes.c_void_p(), ctypes.c_size_t()
+    at = ctypes.c_void_p(stream.cuda_stream)
+    assert hip.hipStreamBeginCapture(at, ctypes.c_int(2)) == 0
+    try:
+        call()
+    finally:
+        assert hip.hipStreamEndCapture(at, ctypes.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("rows", [40, 300, 1024])
+@pytest.mark.parametrize("cols", [5376, 5504, 6144, 7552])
+def test_waves_that_stage_leave_x_its_room(sm, ref, dev, rows, cols):
+    """Two 13-bit codebooks fill 128 of 160 KB of LDS: as many staging waves as
+    fit beside one f32 column, which stays one launch up to 7552 columns."""
+    import torch
+    data = sm.synth_container(rows + cols, rows, cols, 4, 8192, 2, 1)
+    x = torch.from_numpy(np.random.default_rng(cols).standard_normal((1, cols)).astype(np.float32)).to(dev)
+    dc, y, stream = sm.DeviceContainer(data), torch.full((1, rows), float("nan"), device=dev), torch.cuda.Stream()
+    dc.gemv(x, y)
+    torch.cuda.synchronize()
+    assert rel_l2(y[0].cpu().numpy(), ref.decode(data).astype(np.float64) @ x[0].double().cpu().numpy()) <= TIGHT
+    assert launches(stream, lambda: dc.gemv(x, y, stream=stream)) == 1

@@ -321,14 +321,18 @@ __global__ __launch_bounds__(256, 2) void fw_attn_split_kernel(const AttnArgs A)
         const int p = pfirst + kAttnChunk * tile;
         const bool edge = p + kAttnChunk > pos + (DEC ? 0 : 1) || p < allfirst;   /* uniform */
         if (DEC && edge) {
-            /* the last tile: rows from pos on are the new key and value */
+            /* the last tile: row pos is the new key and value. Rows past it
+             * weigh zero, as their scores are masked, and their values are
+             * zero too: the new value again would add 0 times its infinities */
             if (p + c >= pos) {
 #pragma unroll
                 for (int j = 0; j < KQ; j++) kf[s][j] = *(const f4v *) (lkv + d0 + 16 * j + 4 * g);
             }
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++)
-                if (p + 4 * g + ks >= pos) vf[s][ks] = *(const vv *) (lkv + HD + d0 + VW * c);
+            for (int ks = 0; ks < 4; ks++) {
+                const int pp = p + 4 * g + ks;
+                if (pp >= pos) vf[s][ks] = pp == pos ? *(const vv *) (lkv + HD + d0 + VW * c) : (vv) 0.0f;
+            }
         }
         /* this wave's elements of S^T, two chains per block */
         f4v sa[NB], sb[NB];

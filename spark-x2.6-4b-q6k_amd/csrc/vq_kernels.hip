@@ -1399,11 +1399,18 @@ static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
          * the codebooks in one pass of five chunks per thread and stage (and
          * x in two), which the straight-line kernels ask for and the ring
          * form is slow without: waves past the tiles stage and then end. One
-         * f32 column of 1024 x 2560 22.0 -> 8.9 us. As many as LDS holds:
-         * x that fits without them stays in one K range (two 13-bit
-         * codebooks beside one f32 column of 5376 to 7552). */
-        const int wmax = std::max(std::min(10, (n16 + 319) / 320), std::min(10, (c.cols + 1023) / 1024));
-        while (sh.W < wmax && fast_lds(c, nst, S, sh.W + 1) <= (size_t) kLdsMax) sh.W++;
+         * f32 column of 1024 x 2560 22.0 -> 8.9 us. As many as LDS holds
+         * beside x, where that is five or the units are of at most 16 steps:
+         * two 13-bit codebooks and one f32 column of 1024 x 6144 then take
+         * one launch of 6 waves, 14.0 us, and not two of 10 over half of K
+         * each, 24.5 (6656, 4 waves, 13 steps: 21.1 and 35.2). Fewer waves on
+         * longer units lose to the two (6784, 4 waves, 53 steps: 38.0 and
+         * 33.9; 7552, one wave, 59 steps: 70.9 and 38.9), so there the shape
+         * keeps all of its waves, does not fit and K is split. */
+        const int wmax = std::max(sh.W, std::max(std::min(10, (n16 + 319) / 320), std::min(10, (c.cols + 1023) / 1024)));
+        int w = wmax;
+        while (w > sh.W && fast_lds(c, nst, S, w) > (size_t) kLdsMax) w--;
+        sh.W = w >= 5 || M / S / C <= 16 ? w : wmax;
     }
     sh.nwg = 0;
     for (int m = 0; m < c.nmat; m++) sh.nwg += (int) (((c.mats[m].rows * (long) S + 15) / 16 + T - 1) / T);

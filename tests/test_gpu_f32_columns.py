@@ -113,10 +113,10 @@ def launches(stream, call):
 
 
 @pytest.mark.parametrize("rows", [40, 300, 1024])
-@pytest.mark.parametrize("cols", [5376, 5504, 6144, 7552])
-def test_waves_that_stage_leave_x_its_room(sm, ref, dev, rows, cols):
-    """Two 13-bit codebooks fill 128 of 160 KB of LDS: as many staging waves as
-    fit beside one f32 column, which stays one launch up to 7552 columns."""
+@pytest.mark.parametrize("cols,want", [(5376, 1), (5504, 1), (6144, 1), (6656, 1), (6784, 2), (7552, 2), (7680, 2)])
+def test_waves_that_stage_leave_x_its_room(sm, ref, dev, rows, cols, want):
+    """Two 13-bit codebooks fill 128 of 160 KB of LDS: one f32 column stays one
+    launch, with the staging waves that fit beside it, unless few do and units are long."""
     import torch
     data = sm.synth_container(rows + cols, rows, cols, 4, 8192, 2, 1)
     x = torch.from_numpy(np.random.default_rng(cols).standard_normal((1, cols)).astype(np.float32)).to(dev)
@@ -124,4 +124,4 @@ def test_waves_that_stage_leave_x_its_room(sm, ref, dev, rows, cols):
     dc.gemv(x, y)
     torch.cuda.synchronize()
     assert rel_l2(y[0].cpu().numpy(), ref.decode(data).astype(np.float64) @ x[0].double().cpu().numpy()) <= TIGHT
-    assert launches(stream, lambda: dc.gemv(x, y, stream=stream)) == 1
+    assert launches(stream, lambda: dc.gemv(x, y, stream=stream)) == want

@@ -1103,13 +1103,8 @@ static int chain_build(Chain * c) {
 
 template <int W, int R>
 static int chain_launch_w(Chain * c, hipStream_t s) {
-    static int opted[64] = {0};
-    const void * fn = (const void *) vq_chain_kernel<W, R>;
-    if (c->dev >= 0 && c->dev < 64 && !opted[c->dev]) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int) kChainLds);
-        if (e != hipSuccess) return fail_hip("chain LDS opt-in", e);
-        opted[c->dev] = 1;
-    }
+    static LdsAllowed allowed;
+    if (lds_allow(allowed, (const void *) vq_chain_kernel<W, R>, kChainLds, "chain LDS opt-in")) return -1;
     launch_kernel(vq_chain_kernel<W, R>, dim3(c->G), dim3(W * 64), kChainLds, s, (const ChainOp *) c->dops,
                   (const ChainWg *) c->dwgs, (int) c->built_ops.size(), c->flags, c->flags + c->G, c->trace);
     hipError_t e = hipGetLastError();

@@ -20,6 +20,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "lds_allow.h"
+
 namespace sparkmv {
 
 struct Layout {

@@ -43,8 +43,6 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <atomic>
-
 #include <map>
 #include <vector>
 
@@ -2131,13 +2129,10 @@ int prompt_splits(const Model & m, int N, int pos, int window) {
 int prompt_split_launch(const float * qkv, int ldq, int kvd, const float * kc, const float * vc, int pos, int N,
                         int heads, int kv_heads, float scale, int nz, float * po, float * pml, uint32_t * redo,
                         hipStream_t s) {
-    static std::atomic<int> opted{0};
-    if (!opted.load()) {
-        hipError_t e = hipFuncSetAttribute((const void *) fw_attn_prompt_split_kernel,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, kPsLds);
-        if (e != hipSuccess) return fail_hip("LDS opt-in for the split prompt attention", e);
-        opted.store(1);
-    }
+    static LdsAllowed allowed;
+    if (lds_allow(allowed, (const void *) fw_attn_prompt_split_kernel, kPsLds,
+                  "LDS opt-in for the split prompt attention"))
+        return -1;
     hipLaunchKernelGGL(fw_attn_prompt_split_kernel,
                        dim3((unsigned) nz, (unsigned) ((N + kPsTok - 1) / kPsTok), (unsigned) kv_heads), dim3(512),
                        kPsLds, s, qkv, ldq, kvd, kc, vc, pos, N, heads, scale, po, pml, redo);

@@ -824,13 +824,10 @@ static int q6k_rows_per_wave(int cols) {
 template <int NC, int XF32, int RPV>
 static int kq_q6k_staged_k(const uint8_t * bp, int rows, int cols, const void * x, int ldx, int ncol, float * y,
                            int ldy, int accumulate, int rpw, size_t lds, hipStream_t s) {
-    static size_t opted = 0;
-    const void * fn = (const void *) q6k_gemv_staged_kernel<NC, XF32, RPV>;
-    if (lds > 65536 && lds > opted) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
-        if (e != hipSuccess) return fail_hip("LDS opt-in for the staged Q6_K kernel", e);
-        opted = lds;
-    }
+    static LdsAllowed allowed;
+    if (lds_allow(allowed, (const void *) q6k_gemv_staged_kernel<NC, XF32, RPV>, lds,
+                  "LDS opt-in for the staged Q6_K kernel"))
+        return -1;
     /* x waves: enough for one batch of eight 16-byte groups per lane, within 16 waves */
     const int nrw = (rpw + RPV - 1) / RPV;
     int xw = (ncol * cols + 4095) / 4096;
@@ -874,13 +871,10 @@ static int kq_q6k_staged(const uint8_t * bp, int rows, int cols, const void * x,
 template <int NC, int XF32, int PD>
 static int kq_q8_mfma_k(const uint8_t * bp, int rows, int cols, const void * x, int ldx, int ncol, float * y, int ldy,
                         int accumulate, int nwv, int persist, size_t lds, hipStream_t s) {
-    static std::atomic<size_t> opted{0};
-    const void * fn = (const void *) q8_0_mfma_kernel<NC, XF32, PD>;
-    if (lds > 65536 && lds > opted.load()) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
-        if (e != hipSuccess) return fail_hip("LDS opt-in for the matrix-core Q8_0 kernel", e);
-        opted.store(lds);
-    }
+    static LdsAllowed allowed;
+    if (lds_allow(allowed, (const void *) q8_0_mfma_kernel<NC, XF32, PD>, lds,
+                  "LDS opt-in for the matrix-core Q8_0 kernel"))
+        return -1;
     const int ntiles = (rows + 15) / 16;
     int grid = (ntiles + nwv - 1) / nwv;
     if (persist && grid > cu_count()) grid = cu_count();

@@ -712,13 +712,10 @@ static int prefill_rt(int rows, int ntok) {
 
 template <int NST, int EXT, int XF32, int PF, int XT, int RT>
 static int prefill_mfma_rt(const MfmaArgs & P, size_t lds, hipStream_t s) {
-    static size_t opted = 0;
-    const void * fn = (const void *) prefill_mfma_kernel<NST, EXT, XF32, PF, XT, RT>;
-    if (lds > 65536 && lds > opted) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
-        if (e != hipSuccess) return fail_hip("LDS opt-in for the MFMA prefill kernel", e);
-        opted = lds;
-    }
+    static LdsAllowed allowed;
+    if (lds_allow(allowed, (const void *) prefill_mfma_kernel<NST, EXT, XF32, PF, XT, RT>, lds,
+                  "LDS opt-in for the MFMA prefill kernel"))
+        return -1;
     const dim3 grid((unsigned) ((P.rows + RT - 1) / RT), (unsigned) ((P.ntok + kPT - 1) / kPT));
     launch_kernel(prefill_mfma_kernel<NST, EXT, XF32, PF, XT, RT>, grid, dim3(kPThreads), (uint32_t) lds, s, P);
     hipError_t e = hipGetLastError();
@@ -837,14 +834,11 @@ static int cw_workspace(size_t bytes, hipStream_t s, void ** out) {
 
 template <int NST, int EXT, int XF32, int XT, int FOLD>
 static int prefill_cw_tf(const CwArgs & P, int nsplit, hipStream_t s) {
-    static size_t opted = 0;
+    static LdsAllowed allowed;
     const size_t lds = prefill_cw_lds(NST, P.nc);
-    const void * fn = (const void *) prefill_cw_kernel<NST, EXT, XF32, XT, FOLD>;
-    if (lds > 65536 && lds > opted) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
-        if (e != hipSuccess) return fail_hip("LDS opt-in for the codeword prefill kernel", e);
-        opted = lds;
-    }
+    if (lds_allow(allowed, (const void *) prefill_cw_kernel<NST, EXT, XF32, XT, FOLD>, lds,
+                  "LDS opt-in for the codeword prefill kernel"))
+        return -1;
     const dim3 grid((unsigned) ((P.rows + kCR - 1) / kCR), (unsigned) ((P.ntok + kCT - 1) / kCT), (unsigned) nsplit);
     launch_kernel(prefill_cw_kernel<NST, EXT, XF32, XT, FOLD>, grid, dim3(kCThreads), (uint32_t) lds, s, P);
     hipError_t e = hipGetLastError();

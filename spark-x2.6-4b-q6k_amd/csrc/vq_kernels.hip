@@ -1115,7 +1115,7 @@ static int aligned4(const void * p) { return ((uintptr_t) p & 3u) == 0; }
 
 template <int NST, int XF32, int EXT, int MSC, int MC = 0, int XN = 0>
 static int launch_fast_t(const FastArgs & A, int grid, int threads, size_t lds, hipStream_t s) {
-    static size_t opted = 0;
+    static LdsAllowed allowed;
     static std::atomic<int> checked{0};
     const void * fn = (const void *) vq_mfma_kernel<NST, XF32, EXT, MSC, MC, XN>;
     if (!checked.load()) {
@@ -1130,11 +1130,7 @@ static int launch_fast_t(const FastArgs & A, int grid, int threads, size_t lds, 
         }
         checked.store(1);
     }
-    if (lds > 65536 && lds > opted) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
-        if (e != hipSuccess) return fail_hip("LDS opt-in for the VQ block kernel", e);
-        opted = lds;
-    }
+    if (lds_allow(allowed, fn, lds, "LDS opt-in for the VQ block kernel")) return -1;
     launch_kernel(vq_mfma_kernel<NST, XF32, EXT, MSC, MC, XN>, dim3(grid), dim3(threads), (uint32_t) lds, s, A);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail_hip("VQ block kernel launch", e);
@@ -1756,15 +1752,8 @@ static int launch_wave(const VqCall & c, int variant) {
     const int threads = c.threads && c.threads < 256 ? c.threads : 256;
     const int nw = threads / 64;
     const size_t lds = variant == 2 ? (size_t) c.nc * c.dim * 2 : 0;
-    if (lds > 65536) {
-        static size_t opted = 0;
-        if (lds > opted) {
-            hipError_t e = hipFuncSetAttribute((const void *) vq_wave_kernel<1>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
-            if (e != hipSuccess) return fail_hip("LDS opt-in for the codebook wave kernel", e);
-            opted = lds;
-        }
-    }
+    static LdsAllowed allowed;
+    if (lds_allow(allowed, (const void *) vq_wave_kernel<1>, lds, "LDS opt-in for the codebook wave kernel")) return -1;
     for (int m = 0; m < c.nmat; m++) {
         const Layout L = make_layout(c.dim, c.nc, c.mats[m].rows, c.cols, c.v3);
         int grid = c.grid > 0 ? c.grid : (L.rows + nw - 1) / nw;

@@ -140,14 +140,18 @@ __global__ __launch_bounds__(256) void fw_rmsnorm_kernel(const float * x, const 
  * window 0: every position), split by positions over workgroups whose
  * partial results a second launch combines:
  *
- *   fw_attn_split_kernel: workgroup (split, kv head). The window's positions
- *     are cut into tiles of 16 and split s takes `per` consecutive tiles,
- *     per = ceil(tiles / nsplit): one tile each up to 16 * nsplit positions,
- *     so a short window still spreads over the chip, and a long one costs
- *     nsplit partials per head whatever its length. All the columns that read
- *     a kv head's rows run together: column t * G + g is token t (of N) and
- *     query head g of the group's G, at most 32, in NB blocks of 16. So K and
- *     V cross HBM once per call, on the f32 matrix cores.
+ *   fw_attn_split_kernel: workgroup (split, kv head, 16 columns). The window's
+ *     positions are cut into tiles of 16 and split s takes `per` consecutive
+ *     tiles, per = ceil(tiles / nsplit): one tile each up to 16 * nsplit
+ *     positions, so a short window still spreads over the chip, and a long one
+ *     costs nsplit partials per head whatever its length. Columns that read a
+ *     kv head's rows run together on the f32 matrix cores: column t * G + g is
+ *     token t (of N) and query head g of the group's G, at most 32. More than
+ *     16 take a second workgroup, which finds K and V in a cache: both blocks
+ *     in one workgroup was slower in short windows (a block of 8 at position
+ *     20: 8.6 us, 6.4 now; the four-layer call 336 -> 329, 330 with a
+ *     workgroup per 16 positions and token) and in long ones (6001: 22.3 us
+ *     and 19.8).
  *   fw_attn_combine_kernel: per (head, token), rescales the partials to their
  *     overall reference M, divides by L = sum_s l_s e^(m_s - M) and applies the
  *     head's sigmoid gate.
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(256) void fw_rmsnorm_kernel(const float * x, const 
  * wave's matrix time, which a short window needs, and a wave holds only
  * DW / 2 registers per tile of K and V, which lets the next tile be in flight
  * under this one, which a long window needs (two tiles ahead: 45.3 -> 47.0 us
- * at 30000 positions, 22.7 -> 24.9 for the block below).
+ * at 30000 positions).
  *
  * Operand layout (lane 16 g + c), as in the prompt kernel below: a lane
  * reads its K row c as runs of 4 elements (k-step ks contracts element
@@ -192,7 +196,7 @@ __global__ __launch_bounds__(256) void fw_rmsnorm_kernel(const float * x, const 
  * partials combined by four waves per head): one token at position 30007 70 +
  * 56 -> 47 + 4.7 us (partials + combine), at 1003 9.4 + 4.7 -> 7.4 + 4.6, a
  * 512-position window 7.5 + 4.7 -> 6.1 + 4.6; a block of 8 at 6001 79 + 13 ->
- * 22 + 4.0, its 512-position windows 10.2 + 4.8 -> 9.0 + 4.0.
+ * 20 + 4.8, its 512-position windows 10.2 + 4.8 -> 7.9 + 4.1.
  * kAttnSplits: 64 against 128 costs the split kernel 1.7 us at 30007 and saves
  * every combine 0.6; 256 splits 54 + 6.3 at 30007. */
 constexpr int kAttnChunk = 16;     /* positions per tile */
@@ -215,13 +219,13 @@ __host__ __device__ __forceinline__ int attn_per(int n, int nsplit) {
     return (tiles + nsplit - 1) / nsplit;
 }
 
-template <int HD, int NB, int DEC>
+template <int HD, int DEC>
 __global__ __launch_bounds__(256, 2) void fw_attn_split_kernel(const AttnArgs A) {
     constexpr int DW = HD / 4, KQ = DW / 16, VW = DW / 16, QS = HD + 4;
     typedef float f4v __attribute__((ext_vector_type(4)));
     typedef float vv __attribute__((ext_vector_type(VW)));
-    __shared__ __attribute__((aligned(16))) float lq[NB * 16 * QS];
-    __shared__ f4v ls[2][4][NB][64];
+    __shared__ __attribute__((aligned(16))) float lq[16 * QS];
+    __shared__ f4v ls[2][4][64];
     __shared__ __attribute__((aligned(16))) float lkv[DEC ? 2 * HD : 4];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, c = lane & 15;
     const int pos = DEC ? A.st[1] : A.pos0, N = DEC ? 1 : A.N, kvh = blockIdx.y;
@@ -249,8 +253,8 @@ __global__ __launch_bounds__(256, 2) void fw_attn_split_kernel(const AttnArgs A)
     };
     fetch(tb, 0);
     __builtin_amdgcn_sched_barrier(0);
-    /* the queries (rows past the last column repeat it) */
-    const int ncol = N * G;
+    /* the queries (rows past the last column repeat it), from column col0 on */
+    const int ncol = N * G, col0 = DEC ? 0 : 16 * (int) blockIdx.z;
     if constexpr (DEC) {
         /* rotated here (model.rs:416-438): element e < half pairs with
          * e + half, e in [half, 2 half) with e - half */
@@ -283,38 +287,28 @@ __global__ __launch_bounds__(256, 2) void fw_attn_split_kernel(const AttnArgs A)
         }
     } else {
 #pragma unroll
-        for (int k = 0; k < NB * 16 * HD / 4 / 256; k++) {
-            const int i = tid + 256 * k, col = min(i / (HD / 4), ncol - 1), e = 4 * (i & (HD / 4 - 1));
+        for (int k = 0; k < 16 * HD / 4 / 256; k++) {
+            const int i = tid + 256 * k, col = min(col0 + i / (HD / 4), ncol - 1), e = 4 * (i & (HD / 4 - 1));
             const int t = col / G, h = kvh * G + col - t * G;
             *(f4v *) (lq + (i / (HD / 4)) * QS + e) = *(const f4v *) (A.qkv + (size_t) t * A.ldq + (size_t) h * HD + e);
         }
     }
     __syncthreads();
-    float qv[NB][4 * KQ];
-    int pos_t[NB], start_t[NB];
+    const int col = min(col0 + c, ncol - 1);
+    float qv[4 * KQ];
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-        const int col = min(16 * b + c, ncol - 1);
+    for (int j = 0; j < KQ; j++) {
+        const f4v q4 = *(const f4v *) (lq + (DEC ? col : c) * QS + d0 + 16 * j + 4 * g);
 #pragma unroll
-        for (int j = 0; j < KQ; j++) {
-            const f4v q4 = *(const f4v *) (lq + (DEC ? col : 16 * b + c) * QS + d0 + 16 * j + 4 * g);
-#pragma unroll
-            for (int i = 0; i < 4; i++) qv[b][4 * j + i] = q4[i];
-        }
-        pos_t[b] = pos + col / G;
-        start_t[b] = A.window > 0 && pos_t[b] + 1 > A.window ? pos_t[b] + 1 - A.window : 0;
+        for (int i = 0; i < 4; i++) qv[4 * j + i] = q4[i];
     }
+    const int pos_t = pos + col / G, start_t = A.window > 0 && pos_t + 1 > A.window ? pos_t + 1 - A.window : 0;
     /* positions every column sees: the tiles inside need no mask */
     const int allfirst = A.window > 0 && plast + 1 > A.window ? plast + 1 - A.window : 0;
-    f4v o[NB][VW];
-    float m[NB], l[NB];
+    f4v o[VW];
+    float m = -INFINITY, l = 0.0f;
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-        m[b] = -INFINITY;
-        l[b] = 0.0f;
-#pragma unroll
-        for (int r = 0; r < VW; r++) o[b][r] = f4v{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int r = 0; r < VW; r++) o[r] = f4v{0.f, 0.f, 0.f, 0.f};
     auto step = [&](int tile, int s) {
         const int p = pfirst + kAttnChunk * tile;
         const bool edge = p + kAttnChunk > pos + (DEC ? 0 : 1) || p < allfirst;   /* uniform */
@@ -332,57 +326,41 @@ __global__ __launch_bounds__(256, 2) void fw_attn_split_kernel(const AttnArgs A)
                 if (pp >= pos) vf[s][ks] = pp == pos ? *(const vv *) (lkv + HD + d0 + VW * c) : (vv) 0.0f;
             }
         }
-        /* this wave's elements of S^T, two chains per block */
-        f4v sa[NB], sb[NB];
-#pragma unroll
-        for (int b = 0; b < NB; b++) sa[b] = sb[b] = f4v{0.f, 0.f, 0.f, 0.f};
+        /* this wave's elements of S^T, two chains */
+        f4v sa = f4v{0.f, 0.f, 0.f, 0.f}, sb = sa;
 #pragma unroll
         for (int j = 0; j < KQ; j++)
 #pragma unroll
-            for (int i = 0; i < 4; i += 2)
-#pragma unroll
-                for (int b = 0; b < NB; b++) {
-                    sa[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s][j][i], qv[b][4 * j + i], sa[b], 0, 0, 0);
-                    sb[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s][j][i + 1], qv[b][4 * j + i + 1], sb[b], 0, 0, 0);
-                }
-#pragma unroll
-        for (int b = 0; b < NB; b++) ls[s][wave][b][lane] = sa[b] + sb[b];
+            for (int i = 0; i < 4; i += 2) {
+                sa = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s][j][i], qv[4 * j + i], sa, 0, 0, 0);
+                sb = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s][j][i + 1], qv[4 * j + i + 1], sb, 0, 0, 0);
+            }
+        ls[s][wave][lane] = sa + sb;
         __syncthreads();
-        float e[NB][4];
-        bool over = false;
-        float mc[NB];
+        const f4v sc = (ls[s][0][lane] + ls[s][1][lane]) + (ls[s][2][lane] + ls[s][3][lane]);
+        float e[4];
+        float mc = -INFINITY;
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-            const f4v sc = (ls[s][0][b][lane] + ls[s][1][b][lane]) + (ls[s][2][b][lane] + ls[s][3][b][lane]);
-            mc[b] = -INFINITY;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int pp = p + 4 * g + i;
-                e[b][i] = !edge || (pp >= start_t[b] && pp <= pos_t[b]) ? sc[i] * A.scale : -INFINITY;
-                mc[b] = fmaxf(mc[b], e[b][i]);
-            }
-            over = over || mc[b] > m[b] + kPaLag;
+        for (int i = 0; i < 4; i++) {
+            const int pp = p + 4 * g + i;
+            e[i] = !edge || (pp >= start_t && pp <= pos_t) ? sc[i] * A.scale : -INFINITY;
+            mc = fmaxf(mc, e[i]);
         }
-        if (__any(over)) {   /* uniform, and the same in every wave */
+        if (__any(mc > m + kPaLag)) {   /* uniform, and the same in every wave */
+            mc = fmaxf(mc, __shfl_xor(mc, 16, 64));
+            mc = fmaxf(mc, __shfl_xor(mc, 32, 64));
+            const float mn = fmaxf(m, mc);
+            const float a = mn == -INFINITY ? 1.0f : expf(m - mn);   /* nothing seen yet: no rescale */
+            l *= a;
 #pragma unroll
-            for (int b = 0; b < NB; b++) {
-                float x = fmaxf(mc[b], __shfl_xor(mc[b], 16, 64));
-                x = fmaxf(x, __shfl_xor(x, 32, 64));
-                const float mn = fmaxf(m[b], x);
-                const float a = mn == -INFINITY ? 1.0f : expf(m[b] - mn);   /* nothing seen yet: no rescale */
-                l[b] *= a;
-#pragma unroll
-                for (int r = 0; r < VW; r++) o[b][r] *= a;
-                m[b] = mn;
-            }
+            for (int r = 0; r < VW; r++) o[r] *= a;
+            m = mn;
         }
 #pragma unroll
-        for (int b = 0; b < NB; b++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                e[b][i] = e[b][i] == -INFINITY ? 0.0f : expf(e[b][i] - m[b]);
-                l[b] += e[b][i];
-            }
+        for (int i = 0; i < 4; i++) {
+            e[i] = e[i] == -INFINITY ? 0.0f : expf(e[i] - m);
+            l += e[i];
+        }
         if constexpr (!DEC) {
             bool bad = false;
             if (edge) {
@@ -399,15 +377,12 @@ __global__ __launch_bounds__(256, 2) void fw_attn_split_kernel(const AttnArgs A)
                     for (int k = 0; k < 4; k++) {
                         const int pp = p + 4 * q + k;
                         const float * vr = A.vc + (size_t) min(pp, rlast) * kvd + (size_t) kvh * HD + d0 + 4 * VW * g;
+                        const float w = __shfl(e[k], 16 * q + c, 64);
+                        if (pp >= start_t && pp <= pos_t)
 #pragma unroll
-                        for (int b = 0; b < NB; b++) {
-                            const float w = __shfl(e[b][k], 16 * q + c, 64);
-                            if (pp >= start_t[b] && pp <= pos_t[b])
+                            for (int i = 0; i < 4; i++)
 #pragma unroll
-                                for (int i = 0; i < 4; i++)
-#pragma unroll
-                                    for (int r = 0; r < VW; r++) o[b][r][i] += w * vr[VW * i + r];
-                        }
+                                for (int r = 0; r < VW; r++) o[r][i] += w * vr[VW * i + r];
                     }
                 return;
             }
@@ -416,9 +391,7 @@ __global__ __launch_bounds__(256, 2) void fw_attn_split_kernel(const AttnArgs A)
         for (int ks = 0; ks < 4; ks++)
 #pragma unroll
             for (int r = 0; r < VW; r++)
-#pragma unroll
-                for (int b = 0; b < NB; b++)
-                    o[b][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[s][ks][r], e[b][ks], o[b][r], 0, 0, 0);
+                o[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[s][ks][r], e[ks], o[r], 0, 0, 0);
     };
     /* tile t in slot and score buffer (t - tb) & 1, the next one requested
      * before it is worked (past the end the last one again: a branch between
@@ -435,25 +408,21 @@ __global__ __launch_bounds__(256, 2) void fw_attn_split_kernel(const AttnArgs A)
             t++;
         }
     }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (col0 + c >= ncol) return;
+    const int t = col / G, h = kvh * G + col - t * G;
+    const size_t at = ((size_t) t * A.heads + h) * A.nsplit + blockIdx.x;
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-        l[b] += __shfl_xor(l[b], 16, 64);
-        l[b] += __shfl_xor(l[b], 32, 64);
-        const int col = 16 * b + c;
-        if (col >= ncol) continue;
-        const int t = col / G, h = kvh * G + col - t * G;
-        const size_t at = ((size_t) t * A.heads + h) * A.nsplit + blockIdx.x;
+    for (int i = 0; i < 4; i++) {
+        vv v;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            vv v;
-#pragma unroll
-            for (int r = 0; r < VW; r++) v[r] = o[b][r][i];
-            *(vv *) (A.po + at * HD + d0 + VW * (4 * g + i)) = v;
-        }
-        if (wave == 0 && g == 0) {
-            A.pml[2 * at] = m[b];
-            A.pml[2 * at + 1] = l[b];
-        }
+        for (int r = 0; r < VW; r++) v[r] = o[r][i];
+        *(vv *) (A.po + at * HD + d0 + VW * (4 * g + i)) = v;
+    }
+    if (wave == 0 && g == 0) {
+        A.pml[2 * at] = m;
+        A.pml[2 * at + 1] = l;
     }
 }
 
@@ -1886,13 +1855,12 @@ int set_state(Model * m, uint32_t token, int pos, hipStream_t s) {
 int attn_launch(const AttnArgs & A, int hd, int span, const float * gate, int ldg, float * out, uint16_t * out16,
                 bool dec, hipStream_t s) {
     const int tiles = (span + kAttnChunk - 1) / kAttnChunk;
-    const dim3 grid((unsigned) (tiles < A.nsplit ? tiles : A.nsplit), (unsigned) A.kv_heads), b(256);
-    const bool two = A.N * (A.heads / A.kv_heads) > 16;
+    const dim3 grid((unsigned) (tiles < A.nsplit ? tiles : A.nsplit), (unsigned) A.kv_heads,
+                    (unsigned) ((A.N * (A.heads / A.kv_heads) + 15) / 16)), b(256);
 #define FW_ATTN(H)                                                                                                   \
     do {                                                                                                             \
-        if (dec) hipLaunchKernelGGL((fw_attn_split_kernel<H, 1, 1>), grid, b, 0, s, A);                              \
-        else if (two) hipLaunchKernelGGL((fw_attn_split_kernel<H, 2, 0>), grid, b, 0, s, A);                         \
-        else hipLaunchKernelGGL((fw_attn_split_kernel<H, 1, 0>), grid, b, 0, s, A);                                  \
+        if (dec) hipLaunchKernelGGL((fw_attn_split_kernel<H, 1>), grid, b, 0, s, A);                                 \
+        else hipLaunchKernelGGL((fw_attn_split_kernel<H, 0>), grid, b, 0, s, A);                                     \
         hipLaunchKernelGGL(fw_attn_combine_kernel<H / 64>, dim3(A.heads, A.N), dim3(512), 0, s, A, dec ? 1 : 0, gate, \
                            ldg, out, out16);                                                                         \
     } while (0)

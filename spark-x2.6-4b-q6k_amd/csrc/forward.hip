@@ -30,7 +30,7 @@
  * embedding row, rope and the KV row, the attention window. The chain's
  * launches are then the same for every token, so it is recorded once as a
  * HIP graph and replayed per token (sparkmv_model_capture / _replay); each
- * attention launch reserves LDS for its longest window.
+ * attention launch is shaped for its longest window.
  */
 #include "act.h"
 #include "kq.h"
@@ -1704,8 +1704,11 @@ void * sparkmv_model_create(const sparkmv_model_cfg * cfg) {
             return nullptr;
         }
     }
+    /* the interface's limit (sparkmv.h); the kernels here hold kAttnSplits
+     * partials per head whatever the length */
+    constexpr int kMaxCtx = 131072;
+    if (c.max_ctx > kMaxCtx) { set_error("max_ctx %d is above %d", c.max_ctx, kMaxCtx); return nullptr; }
     const long nch_max = ((long) c.max_ctx + kAttnChunk - 1) / kAttnChunk;
-    if (nch_max * 8 > 65536) { set_error("max_ctx %d is above %d", c.max_ctx, 8192 * kAttnChunk); return nullptr; }
     if (c.hidden > 8192) { set_error("hidden %d is above 8192", c.hidden); return nullptr; }
     Model * m = new Model;
     m->c = c;
@@ -2079,10 +2082,13 @@ int block(Model * m, const uint32_t * tokens, int N, int pos, float * logits, hi
 
 /* Span splits of the split-product prompt attention for a chunk, or 0 where
  * it does not run: full layers, four query heads per kv head, and a span of
- * 2048 positions. Below, the partials and two more launches take what the
- * products save (whole prompt call of the four-layer model, 33 tokens at
- * 1500: 1155-1184 us without, 1158-1224 with it; 512 at 2000: 1634-1708 and
- * 1558-1625; 512 at 16384: 2901 and 2050). As many splits as fill the CUs,
+ * 2048 positions, whatever the chunk. Below, the partials and two more
+ * launches take what the products save (whole prompt call of the four-layer
+ * model, 33 tokens at 1500: 1155-1184 us without, 1158-1224 with it). From
+ * there on no chunk is slower: 3, 9, 16 and 64 tokens at 2048 523, 690, 824
+ * and 821 us without, 487, 682, 817 and 818 with it; 3, 9, 16 and 33 at 4096
+ * 586, 604, 678 and 862, and 496, 573, 648 and 843; 9 at 16000 1093 and 936;
+ * 512 at 16384 2901 and 2050. As many splits as fill the CUs,
  * leave a split 256 positions and fit the FFN's buffers. */
 int prompt_splits(const Model & m, int N, int pos, int window) {
     const sparkmv_model_cfg & c = m.c;

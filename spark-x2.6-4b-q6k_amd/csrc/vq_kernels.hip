@@ -332,8 +332,9 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : MC == 2 && XF32 ? 512 :
         /* Several activation columns (speculative verify): codebooks and x
          * are staged in batches of unconditional 16-byte loads (indices past
          * the end re-read the last chunk), then the unit's index words are
-         * requested. The host sends 16-byte aligned x with ldx % 8 == 0 and
-         * at most 5 codebook chunks per thread and stage. */
+         * requested. The host sends x in 16-byte aligned rows (ldx % 8 == 0
+         * for bf16, % 4 for f32) and at most 5 codebook chunks per thread and
+         * stage. */
         typedef uint32_t u4v __attribute__((ext_vector_type(4)));
         typedef uint32_t u4a __attribute__((ext_vector_type(4), aligned(4)));
         constexpr int KS = 5, KXM = 8;
@@ -1659,8 +1660,9 @@ static int launch_fast_part(const VqCall & c, int st0, int nst, int accumulate, 
     }
     const int threads = sh.W * 64;
     A.threads = threads;
-    /* The straight-line kernels take an even codebook, and bf16 x or one
-     * column of f32 x. One column is staged in one branch-free pass and
+    /* The straight-line kernels take an even codebook, and bf16 x, one column
+     * of f32 x, or several that fast_shape_f32 staged (sf; those read from
+     * global memory have xg). One column is staged in one branch-free pass and
      * reduced within a wave: 16-byte aligned x of at most 16 * threads
      * values, one wave per tile, at most 5 codebook chunks per thread and
      * stage. Several columns are staged by loops before the index words

@@ -1308,8 +1308,10 @@ static int straight_ms(int MS, int ext, int norm) {
  * taken where they fit beside the codebooks in one K range, since a value is
  * then split once per workgroup and not once per tile (N = 8 gate+up: 44.2 us
  * with x from global memory, 31.6 in the ring form, 18.9 here). The search is
- * the staged bf16 one over the unit lengths with a kernel. */
-static int fast_shape_f32(const VqCall & c, int nst, FastShape & sh) {
+ * the staged bf16 one over the unit lengths with a kernel. Returns its cost,
+ * or -1. */
+static long fast_shape_f32(const VqCall & c, int nst, FastShape & sh) {
+    sh.ck = 0;
     if (!c.xf32 || c.ncol < 2 || c.nc % 2 || ((uintptr_t) c.x & 15u) || c.ldx % 4) return -1;
     const int M = c.cols / 128, G = cu_count(), n16 = c.nc * 8 / 16;
     long best = -1;
@@ -1335,14 +1337,19 @@ static int fast_shape_f32(const VqCall & c, int nst, FastShape & sh) {
             }
         }
     }
-    return best < 0 ? -1 : 0;
+    return best;
 }
 
 static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
     sh.ck = 0;
     sh.sf = 0;
-    if (fast_shape_f32(c, nst, sh) == 0) return 0;
-    if (kFastXg && fast_shape_xg(c, nst, sh) == 0) {
+    FastShape staged;
+    const long f32_cost = fast_shape_f32(c, nst, staged);
+    if (f32_cost >= 0 && staged.nwg <= cu_count()) {
+        sh = staged;
+        return 0;
+    }
+    if (f32_cost < 0 && kFastXg && fast_shape_xg(c, nst, sh) == 0) {
         /* where x from global memory would take shared tiles (whole tiles
          * leave CUs idle), chunk-split tiles instead: N = 8 down 14.7 ->
          * 13.1-13.6 us, measured; for o (whole tiles on 160 CUs) they gave
@@ -1391,7 +1398,9 @@ static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
     if (T * C > 10) T = 10 / C > 0 ? 10 / C : 1;
     if (T * C > 10) { C = 10; T = 1; }
     sh.S = S; sh.C = C; sh.T = T; sh.W = T * C;
-    if (c.ncol == 1) {
+    sh.nwg = 0;
+    for (int m = 0; m < c.nmat; m++) sh.nwg += (int) (((c.mats[m].rows * (long) S + 15) / 16 + T - 1) / T);
+    if (c.ncol == 1 && (C == 1 || sh.nwg <= G)) {
         /* Short matrices leave a workgroup one to six waves, too few to stage
          * the codebooks in one pass of five chunks per thread and stage (and
          * x in two), which the straight-line kernels ask for and the ring
@@ -1404,13 +1413,12 @@ static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
          * longer units lose to the two (6784, 4 waves, 53 steps: 38.0 and
          * 33.9; 7552, one wave, 59 steps: 70.9 and 38.9), so there the shape
          * keeps all of its waves, does not fit and K is split. */
-        const int wmax = std::max(sh.W, std::max(std::min(10, (n16 + 319) / 320), std::min(10, (c.cols + 1023) / 1024)));
+        const int wstage = std::max(std::min(10, (n16 + 319) / 320), std::min(10, (c.cols + 1023) / 1024));
+        const int wmax = std::max(sh.W, C == 1 ? wstage : std::min(7, wstage));
         int w = wmax;
         while (w > sh.W && fast_lds(c, nst, S, w) > (size_t) kLdsMax) w--;
         sh.W = w >= 5 || M / S / C <= 16 ? w : wmax;
     }
-    sh.nwg = 0;
-    for (int m = 0; m < c.nmat; m++) sh.nwg += (int) (((c.mats[m].rows * (long) S + 15) / 16 + T - 1) / T);
     sh.lds = fast_lds(c, nst, S, sh.W);
     (void) total_rows;
     if (c.ncol > 1) {
@@ -1449,6 +1457,19 @@ static int fast_shape(const VqCall & c, int nst, FastShape & sh) {
                     }
                 }
             }
+        }
+        /* f32 columns whose straight-line units take more than one round of
+         * workgroups: the ring form where its best shape is cheaper by the
+         * same measure, which counts its steps twice. K has no factor there
+         * but 2-step units in many chunks, of one or two tiles a workgroup (3
+         * columns of 3 x 5400 x 3328, 26 steps: 33.9 us in 13 chunks, 25.3 in
+         * the ring form; 8 of 2 x 5744 x 2816, 22 steps: 25.7 and 21.5). In
+         * one round the units win whatever the measure says (4 columns of 2 x
+         * 504 x 2304, 18 steps: 9.7 us and 17.5). */
+        if (f32_cost >= 0) {
+            const int ms = M / sh.S / sh.C;
+            const long ring = (long) (sh.nwg + G - 1) / G * (8 + 2 * ms + sh.C - 1) * 64 + sh.W;
+            if (best < 0 || f32_cost <= ring) sh = staged;
         }
     }
     return 0;

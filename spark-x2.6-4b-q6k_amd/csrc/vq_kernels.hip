@@ -355,7 +355,7 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : MC == 2 && XF32 ? 512 :
          * stage the group's C * MS steps of each part, whose piece cc comes
          * from piece xsrc(cc) of the row */
         constexpr int XP = XF32 ? 4 : 8;           /* columns per 16-byte piece */
-        const int xq = CK ? S * C * MS * 16 : A.cols / XP, nx = XG ? 0 : ncol * xq;
+        const int xq = CK ? S * C * MS * 16 : A.cols >> (XF32 ? 2 : 3), nx = XG ? 0 : ncol * xq;
         auto xsrc = [&](int cc) {
             if constexpr (!CK) return cc;
             const int hh = cc / (C * MS * 16);
@@ -370,7 +370,8 @@ __global__ __launch_bounds__(MC == 1 || MC == 4 ? 1024 : MC == 2 && XF32 ? 512 :
                 const int n = ci[k] / xq, cc = ci[k] - n * xq;
                 /* a slot wholly past x (uniform) would only repeat the last chunk */
                 if (base + k * bd < nx)
-                    xv[k] = *(const u4v *) ((const uint8_t *) A.x + ((size_t) n * A.ldx + XP * xsrc(cc)) * (16 / XP));
+                    xv[k] = XF32 ? *(const u4v *) ((const float *) A.x + (size_t) n * A.ldx + XP * xsrc(cc))
+                                 : *(const u4v *) ((const uint16_t *) A.x + (size_t) n * A.ldx + XP * xsrc(cc));
             }
 #pragma unroll
             for (int k = 0; k < KXM; k++) {

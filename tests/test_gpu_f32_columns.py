@@ -26,10 +26,11 @@ def gemv(sm, dev, data, x, rows, accumulate=None):
 
 
 # (rows, cols, columns, codebook): units of 2, 4, 5 and 10 steps, 13-bit
-# indices, the widest call, ragged rows, and a K (9 steps) that keeps the
-# staged ring kernel
+# indices, the widest call, ragged rows, a K (9 steps) that keeps the staged
+# ring kernel, and two whose 2-step units would take several rounds of workgroups
 F32_COLUMNS = [(6160, 2560, 8, 4096), (300, 2560, 16, 4096), (2560, 10240, 5, 4096), (33, 2560, 8, 4096), (24, 256, 2, 4096), (40, 10240, 16, 4096),
-               (64, 4096, 3, 4096), (48, 4096, 8, 8192), (130, 2560, 7, 4096), (57, 1152, 4, 4096)]
+               (64, 4096, 3, 4096), (48, 4096, 8, 8192), (130, 2560, 7, 4096), (57, 1152, 4, 4096),
+               (5400, 3328, 3, 4096), (5744, 2816, 8, 4096), (504, 2304, 4, 4096)]
 
 
 @pytest.mark.parametrize("rows,cols,ncol,nc", F32_COLUMNS)
@@ -84,7 +85,8 @@ def test_f32_columns_spike_and_non_finite(sm, ref, dev, cols):
 @pytest.mark.parametrize("f32", [False, True], ids=["bf16x", "f32x"])
 @pytest.mark.parametrize("rows,cols,nc", [(1024, 2560, 4096), (8, 256, 4096), (520, 10240, 4096), (16, 10240, 4096),
                                           (1024, 4096, 4096), (600, 1152, 4096), (300, 8192, 8192), (40, 2560, 4094),
-                                          (64, 2560, 1 << 12), (2304, 2304, 4096), (600, 1792, 4096), (70, 1152, 4096), (96, 1152, 8192)])
+                                          (64, 2560, 1 << 12), (2304, 2304, 4096), (600, 1792, 4096), (70, 1152, 4096), (96, 1152, 8192),
+                                          (4300, 9856, 4096), (1984, 2688, 8192)])
 def test_one_column_of_a_short_matrix(sm, ref, dev, rows, cols, nc, f32):
     import torch
     data = sm.synth_container(rows + cols, rows, cols, 4, nc, 2, 1)
